@@ -1537,6 +1537,9 @@ DNOINLINE bool trace_mesh(DTrace &tr, const StDScene &sc, uint32_t mesh_id, bool
     if (COOP) {
         limit = 2u * mesh.triangle_count + 2u;
         if (sc.step_cap && sc.step_cap < limit) limit = sc.step_cap;
+    } else if (limit > ST_ABANDON_DEGENERATE && mesh.triangle_count >= sc.coop_min_tris &&
+               (ray.direction.x == 0 || ray.direction.y == 0 || ray.direction.z == 0)) {
+        limit = ST_ABANDON_DEGENERATE;
     }
     uint32_t steps = 0;
     for (;;) {
