@@ -3,16 +3,18 @@
  * HIP tracing library (gfx950, wave64).
  *
  * Kernels
- *   k_primary_dirs  one lane per traced row and vector component: walks
- *                   the row with the reference's sequential
- *                   `current += right` fp32 sum (render/raytracer.h:156-170)
- *                   and stores the unnormalised `current` vector at every
- *                   ST_DIR_MARK-th pixel (the primary stage finishes the sum
- *                   and normalises it). Rows of every request of a launch
- *                   are flattened into one grid.
- *   k_tile_order    the primary stage's tile claim order: tile order,
- *                   super-tile order, or tiles slower than the mean in the
- *                   previous launch first.
+ *   k_setup         the launch's upload, from page-locked staging, and its
+ *                   cleared counters.
+ *   k_prep          three things by separate blocks. Primary directions: one
+ *                   lane per traced row and vector component walks the row
+ *                   with the reference's sequential `current += right` fp32
+ *                   sum (render/raytracer.h:156-170) and stores the
+ *                   unnormalised `current` vector at every ST_DIR_MARK-th
+ *                   pixel (the primary stage finishes the sum and normalises
+ *                   it); rows of every request of a launch are flattened into
+ *                   one range. The primary stage's tile claim order: tile
+ *                   order, super-tile order, or tiles slower than the mean in
+ *                   the previous launch first. The SSB rects.
  *   k_primary       one wavefront per pixel tile: primary ray, and for
  *   k_primary4      Beauty the first level of the depth loop (shading
  *                   entry, shadow rays, shading; st_wave.h); the same body
@@ -37,6 +39,8 @@
  *                   each pixel's whole path again by a group of blocks,
  *                   with large mesh traversals split across the group.
  *   k_counts        per-request shadow/bounce ray totals.
+ *   k_deliver       window images resolved, grids, hit records and counts
+ *                   written to where the caller wants them.
  */
 #include <hip/hip_runtime.h>
 
@@ -48,6 +52,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <map>
 #include <mutex>
 #include <vector>
 
@@ -107,7 +112,7 @@ struct KReq {
     StDView v;
     uint32_t row_base;     /* first flattened row of this request */
     uint32_t tile_count;
-    uint32_t out_base;     /* first flattened window pixel (display resolve) */
+    uint32_t out_block;    /* first block of the display resolve for this request (k_deliver) */
     uint32_t count_block;  /* first block of k_counts for this request */
     uint32_t *bgra;        /* window image (width1-1)*(height1-1), or NULL */
     uint64_t pad2;
@@ -130,17 +135,15 @@ __device__ static inline uint32_t find_req(const KReq *reqs, uint32_t n, uint32_
     return lo;
 }
 
-/* One lane per traced row and component of the direction: walks that
-   component of the row's sequential `current += right` sum (a vector sum's
-   components are independent fp32 chains, so three lanes run a row's
-   chain a third as long each) and stores the value at every
+/* One lane per traced row and component of the direction (t = 3 * row +
+   component): walks that component of the row's sequential `current += right`
+   sum (a vector sum's components are independent fp32 chains, so three lanes
+   run a row's chain a third as long each) and stores the value at every
    ST_DIR_MARK-th pixel, into the x, y or z word of the pixel's float4
    checkpoint. A pixel's direction is then its checkpoint plus at most
    ST_DIR_MARK - 1 further additions, the same fp32 operations in the same
    order (primary_dir). */
-#define DIRS_BLOCK 192u
-__global__ void __launch_bounds__(DIRS_BLOCK) k_primary_dirs(const KReq *reqs, uint32_t nreq, uint32_t total_rows) {
-    const uint32_t t = blockIdx.x * DIRS_BLOCK + threadIdx.x;
+__device__ static inline void primary_dirs(const KReq *reqs, uint32_t nreq, uint32_t total_rows, uint32_t t) {
     const uint32_t row = t / 3u, c = t - 3u * row;
     if (row >= total_rows) return;
     const uint32_t r = find_req(reqs, nreq, row, true);
@@ -480,7 +483,7 @@ primary_stage(const StDScene *__restrict__ scenes, const KReq *__restrict__ reqs
            scene records load into scalar registers */
         t = __builtin_amdgcn_readfirstlane(t);
         if (t >= total_tiles) break;
-        /* claim order -> tile (k_tile_order) */
+        /* claim order -> tile (order_tiles) */
         t = __builtin_amdgcn_readfirstlane(ldgu(tile_order, t));
         const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
         primary_tile(scenes, reqs, nreq, t, stk, w);
@@ -524,7 +527,7 @@ struct KCoop {
     char *base;            /* group records: group_stride bytes each (CO_HEADER, then the task queue) */
     DCoopSlot *slots;      /* one per block of the launch */
     uint32_t group_stride, q_cap;
-    const uint32_t *epoch; /* launch number (k_tile_order) */
+    const uint32_t *epoch; /* launch number (k_setup) */
 };
 __global__ void __launch_bounds__(REDO_THREADS) k_redo(const StDScene *__restrict__ scenes,
                                                        const KReq *__restrict__ reqs, uint32_t nreq, KWave w,
@@ -645,9 +648,8 @@ __global__ void __launch_bounds__(COST_THREADS) k_cost_total(const uint32_t *__r
    block keeps its tiles in order within each group and claims its ranges
    with one atomic per group (ctr[0] from the front, ctr[1] from the back,
    both zero at launch). Any cost values give a permutation of the tiles,
-   so the order never changes a result. Thread 0 also advances the launch
-   number `epoch` the redo stage tags its cooperative jobs with. */
-#define ORDER_THREADS 1024u
+   so the order never changes a result. */
+#define PREP_THREADS 256u
 #define ORDER_TILE 0u      /* tile order: each request's tiles row by row */
 #define ORDER_HISTORY 1u   /* slowest first, from the previous launch's tile times */
 #define ORDER_SUPER 2u     /* super-tile order */
@@ -669,15 +671,12 @@ __device__ static inline uint32_t super_tile(const KReq *reqs, uint32_t nreq, ui
     return v.tile_base + (band * ST_SUPER + q2 / wc) * w + col * ST_SUPER + q2 % wc;
 }
 
-__global__ void __launch_bounds__(ORDER_THREADS) k_tile_order(const uint32_t *__restrict__ tile_cost,
-                                                              uint32_t *__restrict__ tile_order, uint32_t tiles,
-                                                              const unsigned long long *cost_sum, uint32_t *ctr,
-                                                              uint32_t mode, uint32_t *epoch,
-                                                              const KReq *__restrict__ reqs, uint32_t nreq) {
-    __shared__ uint32_t s_h[ORDER_THREADS / 64], s_l[ORDER_THREADS / 64], s_base[2];
-    const uint32_t i = blockIdx.x * ORDER_THREADS + threadIdx.x;
-    /* a new launch number for the redo stage's group records */
-    if (i == 0) ((ST_GLOBAL uint32_t *)epoch)[0] += 1u;
+__device__ static inline void order_tiles(const uint32_t *__restrict__ tile_cost, uint32_t *__restrict__ tile_order,
+                                          uint32_t tiles, const unsigned long long *cost_sum, uint32_t *ctr,
+                                          uint32_t mode, const KReq *__restrict__ reqs, uint32_t nreq,
+                                          uint32_t block) {
+    __shared__ uint32_t s_h[PREP_THREADS / 64], s_l[PREP_THREADS / 64], s_base[2];
+    const uint32_t i = block * PREP_THREADS + threadIdx.x;
     if (mode != ORDER_HISTORY) {
         if (i < tiles) ((ST_GLOBAL uint32_t *)tile_order)[i] = mode == ORDER_SUPER ? super_tile(reqs, nreq, i) : i;
         return;
@@ -695,7 +694,7 @@ __global__ void __launch_bounds__(ORDER_THREADS) k_tile_order(const uint32_t *__
     }
     __syncthreads();
     uint32_t bh = 0, bl = 0, nh = 0, nl = 0;
-    for (uint32_t k = 0; k < ORDER_THREADS / 64; k++) {
+    for (uint32_t k = 0; k < PREP_THREADS / 64; k++) {
         if (k < wv) { bh += s_h[k]; bl += s_l[k]; }
         nh += s_h[k];
         nl += s_l[k];
@@ -711,7 +710,7 @@ __global__ void __launch_bounds__(ORDER_THREADS) k_tile_order(const uint32_t *__
 
 /* word of the per-launch counters holding the bounce stage's chunk claims */
 #define BOUNCE_CLAIM 32u
-/* words of the per-launch counters holding k_tile_order's two claims */
+/* words of the per-launch counters holding order_tiles's two claims */
 #define ORDER_CLAIM 40u
 
 /* Wave loop over `chunks` chunks of up to 64 queue entries. entry(chunk, lane,
@@ -883,8 +882,7 @@ __global__ void __launch_bounds__(256) k_counts(const KReq *__restrict__ reqs, u
 /* Screen-space bounds on the device (updateSceneSSB, render/SSB.h:137-173),
    one block per request, the same operations as the host pass (st_ssb.h):
    the gate rect of every primitive into the request's rect array. */
-__global__ void __launch_bounds__(256) k_ssb(const StDScene *__restrict__ scenes, const KReq *__restrict__ reqs) {
-    const KReq &q = reqs[blockIdx.x];
+__device__ static inline void ssb_rects(const StDScene *__restrict__ scenes, const KReq &q) {
     if (!q.device_ssb) return;
     const StDView &v = q.v;
     const StDScene sc = scenes[v.scene];
@@ -910,6 +908,32 @@ __global__ void __launch_bounds__(256) k_ssb(const StDScene *__restrict__ scenes
     }
 }
 
+__global__ void __launch_bounds__(256) k_ssb(const StDScene *__restrict__ scenes, const KReq *__restrict__ reqs) {
+    ssb_rects(scenes, reqs[blockIdx.x]);
+}
+
+/* Everything the primary stage needs of a launch besides its upload, in one
+   launch: the primary directions (the longest: a row's additions are one
+   chain, 19 us for 1920), the tile order and the SSB rects, each by its own
+   run of blocks. As three launches one after another they and the gaps
+   between them took PREPB. */
+__global__ void __launch_bounds__(PREP_THREADS) k_prep(const StDScene *__restrict__ scenes,
+                                                       const KReq *__restrict__ reqs, uint32_t nreq,
+                                                       uint32_t total_rows, uint32_t dir_blocks,
+                                                       const uint32_t *__restrict__ tile_cost,
+                                                       uint32_t *__restrict__ tile_order, uint32_t tiles,
+                                                       const unsigned long long *cost_sum, uint32_t *ctr,
+                                                       uint32_t mode, uint32_t order_blocks) {
+    uint32_t b = blockIdx.x;
+    if (b < dir_blocks) {
+        primary_dirs(reqs, nreq, total_rows, b * PREP_THREADS + threadIdx.x);
+    } else if ((b -= dir_blocks) < order_blocks) {
+        order_tiles(tile_cost, tile_order, tiles, cost_sum, ctr, mode, reqs, nreq, b);
+    } else {
+        ssb_rects(scenes, reqs[b - order_blocks]);
+    }
+}
+
 /* Picking (the first-press branch of manipulateSelection,
    viewport/manipulation.h:55-124), one lane per window point: the closed-form
    ray of setRayFromCoords (render/shaders/common.h:170-175), the closest
@@ -922,7 +946,8 @@ struct KPick {
     float rmi[9];                  /* camera rotation_matrix_inverted, rows X, Y, Z */
     uint32_t n;
     const uint32_t *xy;            /* n (x, y) pairs */
-    StPick *out;
+    StPick *out;                   /* page-locked host memory, as is fault: written over the link */
+    uint32_t *fault;               /* set when a traversal ran past its bound */
 };
 
 __global__ void __launch_bounds__(64) k_pick(const StDScene *__restrict__ scenes, const KReq *__restrict__ reqs,
@@ -946,7 +971,7 @@ __global__ void __launch_bounds__(64) k_pick(const StDScene *__restrict__ scenes
     uint32_t type = 0, id = 0;
     bool found = hit_primitives(ray, tr, sc, sc.scene_leaf_ids, sc.prim_count, false, v.rects, (uint16_t)x,
                                 (uint16_t)y);
-    if (tr.abandoned) trav_fault(sc, ST_FAULT_MESH_STEPS);
+    if (tr.abandoned) *(ST_GLOBAL uint32_t *)pk.fault = ST_FAULT_MESH_STEPS;
     if (found) {
         type = hit.object_type;
         id = hit.object_id;
@@ -1000,45 +1025,145 @@ __device__ static inline uint32_t resolve_channel(float c) {
     return s;
 }
 
-__global__ void __launch_bounds__(256) k_resolve(const KReq *reqs, uint32_t nreq, uint32_t total_out) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total_out) return;
-    uint32_t lo = 0, hi = nreq - 1;
-    while (lo < hi) {
-        uint32_t mid = (lo + hi + 1) >> 1;
-        if (reqs[mid].out_base <= i) lo = mid; else hi = mid - 1;
-    }
-    const KReq &r = reqs[lo];
-    if (!r.bgra) return;
+/* Window pixels [at, at + n) of a request's image, n at most 4: neighbours
+   share their corners. */
+__device__ static inline void resolve_pixels(const KReq &r, uint32_t at, uint32_t n) {
     const uint32_t w1 = r.v.width1, w = w1 - 1u;
-    const uint32_t local = i - r.out_base;
-    if (local >= w * (r.v.height1 - 1u)) return;
-    const uint32_t x = local % w, y = local / w;
     const char *base = static_cast<const char *>(r.v.pixels);
-    const size_t tl = (size_t)y * w1 + x, corner[4] = {tl, tl + 1, tl + w1, tl + w1 + 1};
-    float c[4][4];
-    bool background = true;
-    for (int k = 0; k < 4; k++) {
-        /* 24-byte records are 8-byte aligned: three 8-byte loads */
-        const float2 rg = *reinterpret_cast<const float2 *>(base + 24 * corner[k]);
-        const float2 bo = *reinterpret_cast<const float2 *>(base + 24 * corner[k] + 8);
-        const double d = *reinterpret_cast<const double *>(base + 24 * corner[k] + 16);
-        c[k][0] = rg.x; c[k][1] = rg.y; c[k][2] = bo.x; c[k][3] = bo.y;
-        background = background && d == (double)INFINITY;
-    }
-    uint32_t px = 0xFF000000u;
-    if (!background) {
-        uint32_t ch[3];
-        for (int k = 0; k < 3; k++) {
-            float acc = c[3][k] * c[3][3];
-            acc = c[2][k] * c[2][3] + acc;
-            acc = c[1][k] * c[1][3] + acc;
-            acc = c[0][k] * c[0][3] + acc;
-            ch[k] = resolve_channel(acc * 0.25f);
+    uint32_t y = at / w, x = at - y * w;
+    uint32_t out[4];
+    float right[2][4];
+    bool right_background = false;
+    for (uint32_t k = 0; k < n; k++) {
+        const bool fresh = k == 0 || x == 0;   /* the left corners are not the last pixel's right ones */
+        float c[4][4];
+        bool background = true;
+        for (int j = 0; j < 4; j++) {
+            /* TL, TR, BL, BR */
+            if (!(j & 1) && !fresh) {
+                for (int e = 0; e < 4; e++) c[j][e] = right[j >> 1][e];
+                continue;
+            }
+            /* 24-byte records are 8-byte aligned: three 8-byte loads */
+            const char *p = base + 24 * ((size_t)(y + (uint32_t)(j >> 1)) * w1 + x + (uint32_t)(j & 1));
+            const float2 rg = *reinterpret_cast<const float2 *>(p);
+            const float2 bo = *reinterpret_cast<const float2 *>(p + 8);
+            const double d = *reinterpret_cast<const double *>(p + 16);
+            c[j][0] = rg.x; c[j][1] = rg.y; c[j][2] = bo.x; c[j][3] = bo.y;
+            const bool far = d == (double)INFINITY;
+            if (j & 1) {
+                for (int e = 0; e < 4; e++) right[j >> 1][e] = c[j][e];
+                background = background && far;
+            } else {
+                right_background = j == 0 ? far : right_background && far;
+            }
         }
-        px |= ch[2] | (ch[1] << 8) | (ch[0] << 16);
+        /* right_background: so far the left corners' (the last pixel's right ones) */
+        const bool all = background && right_background;
+        right_background = background;
+        uint32_t px = 0xFF000000u;
+        if (!all) {
+            uint32_t ch[3];
+            for (int e = 0; e < 3; e++) {
+                float acc = c[3][e] * c[3][3];
+                acc = c[2][e] * c[2][3] + acc;
+                acc = c[1][e] * c[1][3] + acc;
+                acc = c[0][e] * c[0][3] + acc;
+                ch[e] = resolve_channel(acc * 0.25f);
+            }
+            px |= ch[2] | (ch[1] << 8) | (ch[0] << 16);
+        }
+        out[k] = px;
+        if (++x == w) { x = 0; y++; }
     }
-    r.bgra[local] = px;
+    uint32_t *o = r.bgra + at;
+    if (n == 4u && ((uintptr_t)o & 15u) == 0) {
+        *reinterpret_cast<uint4 *>(o) = make_uint4(out[0], out[1], out[2], out[3]);
+    } else {
+        for (uint32_t k = 0; k < n; k++) o[k] = out[k];
+    }
+}
+
+/* What a launch hands over, in one launch at its end: window images (the
+   display resolve, straight to where they go), traced grids and hit records
+   (16 KB of a segment per block), and the ray counts. Destinations are
+   page-locked host memory that the device writes over the link, or device
+   buffers that are copied on from there. Bound by the link (50 of its 57 GB/s):
+   160 window images, 189 MB, take 3.8 ms; resolved into device memory
+   (0.7 ms) and copied by a call each they took 7. */
+#define DELIVER_THREADS 256u
+#define RESOLVE_PIXELS (4u * DELIVER_THREADS)   /* per block */
+#define SEG_CHUNK 16384u
+struct KSeg {
+    const char *src;
+    char *dst;
+    uint64_t bytes;        /* a multiple of 4, as are both addresses */
+    uint32_t first_block;
+    uint32_t pad;
+};
+__device__ static inline void copy_segment(const KSeg &g, uint32_t chunk) {
+    const uint64_t at = (uint64_t)chunk * SEG_CHUNK;
+    const uint32_t n = (uint32_t)min((uint64_t)SEG_CHUNK, g.bytes - at);
+    const char *src = g.src + at;
+    char *dst = g.dst + at;
+    if ((((uintptr_t)src | (uintptr_t)dst) & 15u) == 0) {
+        for (uint32_t i = threadIdx.x * 16u; i + 16u <= n; i += DELIVER_THREADS * 16u)
+            *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(src + i);
+        const uint32_t tail = n & ~15u;
+        for (uint32_t i = tail + threadIdx.x * 4u; i < n; i += DELIVER_THREADS * 4u)
+            *reinterpret_cast<uint32_t *>(dst + i) = *reinterpret_cast<const uint32_t *>(src + i);
+    } else {
+        for (uint32_t i = threadIdx.x * 4u; i < n; i += DELIVER_THREADS * 4u)
+            *reinterpret_cast<uint32_t *>(dst + i) = *reinterpret_cast<const uint32_t *>(src + i);
+    }
+}
+__global__ void __launch_bounds__(DELIVER_THREADS) k_deliver(const KReq *__restrict__ reqs, uint32_t nreq,
+                                                             uint32_t resolve_blocks, const KSeg *__restrict__ segs,
+                                                             uint32_t nseg, uint32_t seg_blocks,
+                                                             const unsigned long long *counts,
+                                                             unsigned long long *counts_out, uint32_t ncounts) {
+    uint32_t b = blockIdx.x;
+    if (b < resolve_blocks) {
+        uint32_t lo = 0, hi = nreq - 1;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1) >> 1;
+            if (reqs[mid].out_block <= b) lo = mid; else hi = mid - 1;
+        }
+        const KReq &r = reqs[lo];
+        const uint32_t at = (b - r.out_block) * RESOLVE_PIXELS + 4u * threadIdx.x;
+        const uint32_t total = r.bgra ? (r.v.width1 - 1u) * (r.v.height1 - 1u) : 0u;
+        if (at < total) resolve_pixels(r, at, min(4u, total - at));
+    } else if ((b -= resolve_blocks) < seg_blocks) {
+        uint32_t lo = 0, hi = nseg - 1;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1) >> 1;
+            if (segs[mid].first_block <= b) lo = mid; else hi = mid - 1;
+        }
+        copy_segment(segs[lo], b - segs[lo].first_block);
+    } else {
+        for (uint32_t i = threadIdx.x; i < ncounts; i += DELIVER_THREADS) counts_out[i] = counts[i];
+    }
+}
+
+/* A launch's upload and cleared words, by a kernel that reads the page-locked
+   staging over the link: one launch instead of a copy and three fills. Thread
+   0 also advances the launch number `epoch` that the redo stage tags its
+   cooperative jobs with. Every block clears its share. */
+#define SETUP_THREADS 256u
+__global__ void __launch_bounds__(SETUP_THREADS) k_setup(const uint4 *__restrict__ src, uint4 *__restrict__ dst,
+                                                         uint32_t n16, unsigned long long *counts, uint32_t ncounts,
+                                                         uint32_t *claims, uint32_t nclaims, uint32_t *queue_ctr,
+                                                         uint32_t *epoch) {
+    const uint32_t t = blockIdx.x * SETUP_THREADS + threadIdx.x, threads = gridDim.x * SETUP_THREADS;
+    for (uint32_t i = t; i < n16; i += threads) dst[i] = src[i];
+    for (uint32_t i = t; i < ncounts; i += threads) counts[i] = 0;
+    for (uint32_t i = t; i < nclaims; i += threads) claims[i] = 0;
+    if (queue_ctr && t < 2u) queue_ctr[t] = 0;
+    if (epoch && t == 0) epoch[0] += 1u;
+}
+static uint32_t setup_blocks(size_t bytes) {
+    const size_t b = (bytes / 16 + SETUP_THREADS - 1) / SETUP_THREADS;
+    return (uint32_t)(b < 4 ? 4 : b > 512 ? 512 : b);
 }
 
 __global__ void k_zero_u32(uint32_t *p, uint32_t n) {
@@ -1048,6 +1173,25 @@ __global__ void k_zero_u32(uint32_t *p, uint32_t n) {
 __global__ void k_zero_u64(unsigned long long *p, uint32_t n) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0;
+}
+
+/* ---- page-locked host memory ---------------------------------------------- */
+
+/* The library's live page-locked blocks (st_host_alloc), by address: outputs
+   inside one are written by the device itself (k_deliver). */
+static std::mutex g_pin_mu;
+static std::map<uintptr_t, size_t> &g_pinned = *new std::map<uintptr_t, size_t>;   /* lives as long as the process */
+
+static bool pinned_range(const void *p, size_t bytes) {
+    std::lock_guard<std::mutex> lk(g_pin_mu);
+    auto it = g_pinned.upper_bound((uintptr_t)p);
+    if (it == g_pinned.begin()) return false;
+    --it;
+    return (uintptr_t)p + bytes <= it->first + it->second;
+}
+/* an output that k_deliver can write: page-locked, and of 4-byte words */
+static bool deliverable(const void *p, size_t bytes) {
+    return ((uintptr_t)p & 3u) == 0 && (bytes & 3u) == 0 && pinned_range(p, bytes);
 }
 
 /* ---- context ------------------------------------------------------------ */
@@ -1068,15 +1212,16 @@ struct LaunchCtx {
     hipStream_t stream;
     Arena work;            /* per-launch device buffers (grow-only) */
     char *staging;         /* pinned host staging: uploads, then the ray-count readback */
+    char *staging_dev;     /* the same memory at the device's address */
     size_t staging_cap;
     uint32_t *tile_cost;   /* [tile_cap] each tile's time in the last primary stage */
-    uint32_t *tile_order;  /* [tile_cap] the primary stage's claim order (k_tile_order) */
+    uint32_t *tile_order;  /* [tile_cap] the primary stage's claim order (order_tiles) */
     uint32_t tile_cap;
     uint64_t tile_sig;     /* shape of the launch whose times tile_cost holds (0: none) */
     unsigned long long *cost_sum; /* sum of tile_cost over the last launch (k_cost_total) */
     uint32_t *tile_counter; /* CLAIM_WORDS words zeroed per launch: [0] the persistent primary stage's
                                tile counter, [BOUNCE_CLAIM] the bounce stage's chunk claims (128 B
-                               apart), [ORDER_CLAIM] k_tile_order's, [XCD_CLAIM + 32k] chunk k's */
+                               apart), [ORDER_CLAIM] order_tiles's, [XCD_CLAIM + 32k] chunk k's */
     hipEvent_t ev[4];
     int stage_timing;      /* record an event after every stage launch */
     int graph_mode;        /* capture launches into a graph, replay while the launch shape repeats */
@@ -1133,8 +1278,8 @@ static char *g_noalloc_scratch[ST_MAX_DEVICES];
 /* host side of a st_render_noalloc launch: the upload block (request,
    scene record, row starts) and the ray counts read back */
 #define ST_NOALLOC_HOST_BYTES (1u << 21)
-static char g_noalloc_host[ST_NOALLOC_HOST_BYTES] __attribute__((aligned(256)));
-static unsigned long long g_noalloc_counts[5];
+static char *g_noalloc_host, *g_noalloc_host_dev;   /* page-locked, taken by st_init; its device address */
+#define ST_NOALLOC_COUNTS (ST_NOALLOC_HOST_BYTES - 256u)   /* the counts' place in it */
 
 static int ctx_init(LaunchCtx *c) {
     HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
@@ -1214,6 +1359,11 @@ extern "C" int st_init(int device) {
     void *sp = NULL;
     HIP_TRY(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
     g_noalloc_scratch[device] = (char *)sp;
+    void *hp = NULL, *hd = NULL;
+    HIP_TRY(hipHostMalloc(&hp, ST_NOALLOC_HOST_BYTES, hipHostMallocDefault));
+    HIP_TRY(hipHostGetDevicePointer(&hd, hp, 0));
+    g_noalloc_host = (char *)hp;
+    g_noalloc_host_dev = (char *)hd;
     g.device = device;
     g.ready = 1;
     return ST_OK;
@@ -1268,10 +1418,13 @@ static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 static int staging_reserve(LaunchCtx *c, size_t bytes) {
     if (c->staging_cap >= bytes) return ST_OK;
     if (c->staging) HIP_TRY(hipHostFree(c->staging));
-    c->staging = NULL;
+    c->staging = c->staging_dev = NULL;
     c->staging_cap = 0;
     size_t cap = bytes + bytes / 4 + 65536;
     HIP_TRY(hipHostMalloc((void **)&c->staging, cap, hipHostMallocDefault));
+    void *dev = NULL;
+    HIP_TRY(hipHostGetDevicePointer(&dev, c->staging, 0));
+    c->staging_dev = (char *)dev;
     c->staging_cap = cap;
     return ST_OK;
 }
@@ -1734,6 +1887,10 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
     uint32_t rows = 0, tiles = 0;
     uint64_t out_px = 0;
     std::vector<uint64_t> shape = {n, tune.tile_shift};
+    /* outputs that the device writes itself (page-locked); the others are
+       copied on after the launch */
+    std::vector<char> own_px(n), own_hits(n), own_bgra(n);
+    uint32_t nseg = 0, seg_blocks = 0, resolve_blocks = 0;
     for (uint32_t i = 0; i < n; i++) {
         StSceneHandle *s = scenes[i];
         if (!s || !s->host || !s->dbuf) return set_err(ST_ERR_ARG, "request %u has no resident scene", i);
@@ -1746,8 +1903,13 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
                        (want_hits ? round256(px * 16) : 0);
         if (bgra_host && bgra_host[i]) {
             if (hv[i].dv.width1 < 2 || hv[i].dv.height1 < 2) return set_err(ST_ERR_ARG, "request %u: empty window", i);
-            per_req_out += round256((size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4);
+            const size_t wb = (size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4;
+            own_bgra[i] = deliverable(bgra_host[i], wb);
+            if (!own_bgra[i]) per_req_out += round256(wb);
         }
+        own_px[i] = pixels_host && pixels_host[i] && deliverable(pixels_host[i], px * 24);
+        own_hits[i] = want_hits && hits_host && hits_host[i] && deliverable(hits_host[i], px * 16);
+        nseg += (uint32_t)own_px[i] + (uint32_t)own_hits[i];
         const uint32_t tw = 1u << tune.tile_shift, th = 64u >> tune.tile_shift;
         hv[i].dv.tile_shift = tune.tile_shift;
         hv[i].dv.tiles_x = (hv[i].dv.width1 + tw - 1) / tw;
@@ -1770,6 +1932,8 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
         rect_off[i] = up;
         up += round256((scenes[i]->host->prim_count + 1) * 16ull);
     }
+    const size_t o_segs = up;
+    up += round256(nseg * sizeof(KSeg));
     /* wavefront buffers of the Beauty depth loop: levels = largest depth,
        shadow planes = largest light count among Beauty requests */
     uint32_t levels = 0, lmax = 1;
@@ -1862,7 +2026,12 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
         sc_h[k].spill_s = spill_s;
         sc_h[k].spill_m = spill_m;
     }
-    uint32_t row_base = 0, out_base = 0, count_blocks = 0, any_device_ssb = 0;
+    uint32_t row_base = 0, count_blocks = 0, any_device_ssb = 0, seg = 0;
+    KSeg *segs_h = (KSeg *)(st + o_segs);
+    auto deliver = [&](const void *src, void *dst, size_t bytes) {
+        segs_h[seg++] = KSeg{(const char *)src, (char *)dst, bytes, seg_blocks, 0};
+        seg_blocks += (uint32_t)((bytes + SEG_CHUNK - 1) / SEG_CHUNK);
+    };
     for (uint32_t i = 0; i < n; i++) {
         size_t px = (size_t)hv[i].dv.width1 * hv[i].dv.height1;
         StDView &dv = hv[i].dv;
@@ -1879,12 +2048,17 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
         memset(&reqs_h[i], 0, sizeof(KReq));
         reqs_h[i].v = dv;
         reqs_h[i].row_base = row_base;
-        reqs_h[i].out_base = out_base;
+        reqs_h[i].out_block = resolve_blocks;
         reqs_h[i].tile_count = dv.tiles_x * ((dv.height1 + (64u >> dv.tile_shift) - 1) / (64u >> dv.tile_shift));
         reqs_h[i].count_block = count_blocks;
         count_blocks += (reqs_h[i].tile_count + COUNT_TILES - 1) / COUNT_TILES;
-        uint32_t wpx = (dv.width1 - 1) * (dv.height1 - 1);
-        reqs_h[i].bgra = (bgra_host && bgra_host[i]) ? (uint32_t *)arena_take(&c->work, (size_t)wpx * 4) : NULL;
+        const uint32_t wpx = (dv.width1 - 1) * (dv.height1 - 1);
+        if (bgra_host && bgra_host[i]) {
+            reqs_h[i].bgra = own_bgra[i] ? bgra_host[i] : (uint32_t *)arena_take(&c->work, (size_t)wpx * 4);
+            resolve_blocks += (wpx + RESOLVE_PIXELS - 1) / RESOLVE_PIXELS;
+        }
+        if (own_px[i]) deliver(dv.pixels, pixels_host[i], px * 24);
+        if (own_hits[i]) deliver(dv.hits, hits_host[i], px * 16);
         if (hv[i].device_ssb) {
             const sm3 &m = hv[i].rotation_matrix_inverted;
             const float rmi[9] = {m.X.x, m.X.y, m.X.z, m.Y.x, m.Y.y, m.Y.z, m.Z.x, m.Z.y, m.Z.z};
@@ -1894,7 +2068,6 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
             any_device_ssb = 1;
         }
         row_base += dv.height1;
-        out_base += wpx;
     }
     KWave w;
     memset(&w, 0, sizeof w);
@@ -1964,6 +2137,7 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
     }
     const uint32_t cost_blocks = std::min<uint32_t>((tiles + COST_THREADS - 1) / COST_THREADS, 1024u);
 
+    const bool timed = kernel_ms != NULL;
     /* per-stage timing (bench): an event before the first stage and after each */
     uint32_t marks = 0;
     const bool graph = c->graph_mode != 0;
@@ -1979,30 +2153,25 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
        what a graph captures. ev[0] .. ev[1] brackets every kernel of the
        launch (the render time st_render_timed reports). */
     auto enqueue = [&]() -> int {
-        HIP_TRY(hipMemcpyAsync(blk, st, up, hipMemcpyHostToDevice, c->stream));
-        if (!graph) HIP_TRY(hipEventRecord(c->ev[0], c->stream));
-        hipLaunchKernelGGL(k_zero_u64, dim3((3 * n + 2 + 255) / 256), dim3(256), 0, c->stream, cnt_d, 3 * n + 2);
-        hipLaunchKernelGGL(k_zero_u32, dim3(CLAIM_WORDS / 256u), dim3(256), 0, c->stream, c->tile_counter,
-                           CLAIM_WORDS);
+        hipLaunchKernelGGL(k_setup, dim3(setup_blocks(up)), dim3(SETUP_THREADS), 0, c->stream,
+                           (const uint4 *)c->staging_dev, (uint4 *)blk, (uint32_t)(up / 16), cnt_d, 3 * n + 2,
+                           c->tile_counter, CLAIM_WORDS, w.ctr, (uint32_t *)(c->cost_sum + 1));
         static_assert(BOUNCE_CLAIM < ORDER_CLAIM && ORDER_CLAIM + 1 < XCD_CLAIM &&
-                          XCD_CLAIM + 8 * XCD_CLAIM_STRIDE <= CLAIM_WORDS && CLAIM_WORDS % 256u == 0,
+                          XCD_CLAIM + 8 * XCD_CLAIM_STRIDE <= CLAIM_WORDS,
                       "claim counters share the zeroed words");
-        if (any_device_ssb)
-            hipLaunchKernelGGL(k_ssb, dim3(n), dim3(256), 0, c->stream, (const StDScene *)sc_d, (const KReq *)reqs_d);
-        if (levels)
-            hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, c->stream, w.ctr, 2u);
-        hipLaunchKernelGGL(k_primary_dirs, dim3((uint32_t)(((uint64_t)rows * 3 + DIRS_BLOCK - 1) / DIRS_BLOCK)),
-                           dim3(DIRS_BLOCK), 0, c->stream, reqs_d, n, rows);
-        HIP_TRY(hipGetLastError());
+        if (!graph && timed) HIP_TRY(hipEventRecord(c->ev[0], c->stream));
         if (use_history) {
             hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, c->cost_sum, 1u);
             hipLaunchKernelGGL(k_cost_total, dim3(cost_blocks), dim3(COST_THREADS), 0, c->stream,
                                (const uint32_t *)c->tile_cost, tiles, c->cost_sum);
         }
-        hipLaunchKernelGGL(k_tile_order, dim3((tiles + ORDER_THREADS - 1) / ORDER_THREADS), dim3(ORDER_THREADS), 0,
-                           c->stream, (const uint32_t *)c->tile_cost, c->tile_order, tiles,
+        const uint32_t dir_blocks = (uint32_t)(((uint64_t)rows * 3 + PREP_THREADS - 1) / PREP_THREADS);
+        const uint32_t order_blocks = (tiles + PREP_THREADS - 1) / PREP_THREADS;
+        hipLaunchKernelGGL(k_prep, dim3(dir_blocks + order_blocks + (any_device_ssb ? n : 0u)), dim3(PREP_THREADS), 0,
+                           c->stream, (const StDScene *)sc_d, (const KReq *)reqs_d, n, rows, dir_blocks,
+                           (const uint32_t *)c->tile_cost, c->tile_order, tiles,
                            (const unsigned long long *)c->cost_sum, c->tile_counter + ORDER_CLAIM, order_mode,
-                           (uint32_t *)(c->cost_sum + 1), (const KReq *)reqs_d, n);
+                           order_blocks);
         HIP_TRY(hipGetLastError());
         HIP_TRY(mark());
         if (waves4)
@@ -2046,7 +2215,7 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
             hipLaunchKernelGGL(k_counts, dim3(count_blocks), dim3(256), 0, c->stream, (const KReq *)reqs_d, n,
                                (const uint32_t *)w.counts);
         HIP_TRY(hipGetLastError());
-        if (!graph) HIP_TRY(hipEventRecord(c->ev[1], c->stream));
+        if (!graph && timed) HIP_TRY(hipEventRecord(c->ev[1], c->stream));
         return ST_OK;
     };
 
@@ -2094,30 +2263,29 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
             c->graph_sig = sig;
             g.graph_captures++;
         }
-        HIP_TRY(hipEventRecord(c->ev[0], c->stream));
+        if (timed) HIP_TRY(hipEventRecord(c->ev[0], c->stream));
         HIP_TRY(hipGraphLaunch(c->graph_exec, c->stream));
-        HIP_TRY(hipEventRecord(c->ev[1], c->stream));
+        if (timed) HIP_TRY(hipEventRecord(c->ev[1], c->stream));
         g.graph_launches++;
     }
     /* this launch's tile times are now what tile_cost will hold */
     c->tile_sig = tile_sig;
-    if (bgra_host && out_px) {
-        hipLaunchKernelGGL(k_resolve, dim3((uint32_t)((out_px + 255) / 256)), dim3(256), 0, c->stream,
-                           (const KReq *)reqs_d, n, (uint32_t)out_px);
-        HIP_TRY(hipGetLastError());
-    }
+    hipLaunchKernelGGL(k_deliver, dim3(resolve_blocks + seg_blocks + 1), dim3(DELIVER_THREADS), 0, c->stream,
+                       (const KReq *)reqs_d, n, resolve_blocks, (const KSeg *)(blk + o_segs), nseg, seg_blocks,
+                       (const unsigned long long *)cnt_d, (unsigned long long *)(c->staging_dev + o_readback),
+                       3 * n + 2);
+    HIP_TRY(hipGetLastError());
     for (uint32_t i = 0; i < n; i++) {
         size_t px = (size_t)hv[i].dv.width1 * hv[i].dv.height1;
-        if (pixels_host && pixels_host[i])
+        if (pixels_host && pixels_host[i] && !own_px[i])
             HIP_TRY(hipMemcpyAsync(pixels_host[i], reqs_h[i].v.pixels, px * 24, hipMemcpyDeviceToHost, c->stream));
-        if (hits_host && hits_host[i] && want_hits)
+        if (hits_host && hits_host[i] && want_hits && !own_hits[i])
             HIP_TRY(hipMemcpyAsync(hits_host[i], reqs_h[i].v.hits, px * 16, hipMemcpyDeviceToHost, c->stream));
-        if (reqs_h[i].bgra)
+        if (reqs_h[i].bgra && !own_bgra[i])
             HIP_TRY(hipMemcpyAsync(bgra_host[i], reqs_h[i].bgra,
                                    (size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4, hipMemcpyDeviceToHost,
                                    c->stream));
     }
-    HIP_TRY(hipMemcpyAsync(cnt_h, cnt_d, cnt_bytes, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->last_redo = (uint32_t)cnt_h[3 * (size_t)n + 1];
     if (cnt_h[3 * (size_t)n])
@@ -2204,7 +2372,8 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
        counts + fault word, direction checkpoints, frame, hit records, tile
        claim order, tile times, counters, depth-loop state */
     const size_t o_scene = round256(sizeof(KReq)), o_rows = o_scene + round256(sizeof(StDScene));
-    const size_t o_rects = o_rows + round256((size_t)height1 * 16), up_host = o_rects;
+    const size_t o_segs = o_rows + round256((size_t)height1 * 16);
+    const size_t o_rects = o_segs + round256(2 * sizeof(KSeg)), up_host = o_rects;
     size_t off = o_rects + round256(((size_t)P + 1) * 16);
     auto take = [&](size_t bytes) {
         const size_t o = off;
@@ -2238,7 +2407,7 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
         return set_err(ST_ERR_MEMORY, "request needs %zu bytes of scratch; st_render_noalloc has %u", off + 256,
                        (unsigned)ST_NOALLOC_SCRATCH_BYTES);
     uint32_t *const epoch = (uint32_t *)(base + ST_NOALLOC_SCRATCH_BYTES - 256);
-    if (up_host > ST_NOALLOC_HOST_BYTES) return set_err(ST_ERR_ARG, "view too tall for st_render_noalloc");
+    if (up_host > ST_NOALLOC_COUNTS) return set_err(ST_ERR_ARG, "view too tall for st_render_noalloc");
     StHostView hv;
     if (st_view_prepare_rows(hs, view, &hv, (float *)(g_noalloc_host + o_rows)))
         return set_err(ST_ERR_ARG, "invalid view");
@@ -2258,7 +2427,7 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
     unsigned long long *cnt_d = (unsigned long long *)(base + o_cnt);
     dv.counters = cnt_d;
     rq->row_base = 0;
-    rq->out_base = 0;
+    rq->out_block = 0;
     rq->tile_count = tiles;
     rq->count_block = 0;
     const sm3 &m = hv.rotation_matrix_inverted;
@@ -2307,23 +2476,30 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
         if (tune.blocks_per_cu < 4)
             (void)capped_blocks(reinterpret_cast<const void *>(k_primary), lds, tune.blocks_per_cu, &lds_primary);
     }
+    /* page-locked outputs are written by the device itself */
+    const bool own_px = deliverable(pixels, px * 24), own_hits = hits && deliverable(hits, px * 16);
+    uint32_t nseg = 0, seg_blocks = 0;
+    auto deliver = [&](size_t src, void *dst, size_t bytes) {
+        ((KSeg *)(g_noalloc_host + o_segs))[nseg++] = KSeg{base + src, (char *)dst, bytes, seg_blocks, 0};
+        seg_blocks += (uint32_t)((bytes + SEG_CHUNK - 1) / SEG_CHUNK);
+    };
+    if (own_px) deliver(o_pix, pixels, px * 24);
+    if (own_hits) deliver(o_hits, hits, px * 16);
     const KReq *reqs_d = (const KReq *)base;
     const StDScene *sc_d = (const StDScene *)(base + o_scene);
     uint32_t *ctr = (uint32_t *)(base + o_ctr);
     hipStream_t stream = g.main.stream;
     /* the request, scene record and row starts; the rects region is filled
        by the device SSB pass */
-    HIP_TRY(hipMemcpyAsync(base, g_noalloc_host, up_host, hipMemcpyHostToDevice, stream));
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, stream, cnt_d, 5u);
-    hipLaunchKernelGGL(k_zero_u32, dim3(CLAIM_WORDS / 256u), dim3(256), 0, stream, ctr, CLAIM_WORDS);
-    hipLaunchKernelGGL(k_ssb, dim3(1), dim3(256), 0, stream, sc_d, reqs_d);
-    if (beauty) hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, stream, w.ctr, 2u);
-    hipLaunchKernelGGL(k_primary_dirs, dim3((height1 * 3 + DIRS_BLOCK - 1) / DIRS_BLOCK), dim3(DIRS_BLOCK), 0, stream,
-                       reqs_d, 1u, height1);
-    hipLaunchKernelGGL(k_tile_order, dim3((tiles + ORDER_THREADS - 1) / ORDER_THREADS), dim3(ORDER_THREADS), 0, stream,
-                       (const uint32_t *)(base + o_cost), (uint32_t *)(base + o_order), tiles,
+    hipLaunchKernelGGL(k_setup, dim3(setup_blocks(up_host)), dim3(SETUP_THREADS), 0, stream,
+                       (const uint4 *)g_noalloc_host_dev, (uint4 *)base, (uint32_t)(up_host / 16), cnt_d, 5u, ctr,
+                       CLAIM_WORDS, beauty ? w.ctr : NULL, epoch);
+    const uint32_t dir_blocks = (height1 * 3 + PREP_THREADS - 1) / PREP_THREADS;
+    const uint32_t order_blocks = (tiles + PREP_THREADS - 1) / PREP_THREADS;
+    hipLaunchKernelGGL(k_prep, dim3(dir_blocks + order_blocks + 1), dim3(PREP_THREADS), 0, stream, sc_d, reqs_d, 1u,
+                       height1, dir_blocks, (const uint32_t *)(base + o_cost), (uint32_t *)(base + o_order), tiles,
                        (const unsigned long long *)cnt_d, ctr + ORDER_CLAIM,
-                       tune.cost_order == 2u ? ORDER_SUPER : ORDER_TILE, epoch, reqs_d, 1u);
+                       tune.cost_order == 2u ? ORDER_SUPER : ORDER_TILE, order_blocks);
     HIP_TRY(hipGetLastError());
     hipLaunchKernelGGL(k_primary, dim3(blocks), dim3(BLOCK_THREADS), lds_primary, stream, sc_d, reqs_d, 1u, tiles, ctr,
                        claim_mode, xcd_blocks, ks, km, w,
@@ -2340,17 +2516,21 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
         hipLaunchKernelGGL(k_counts, dim3((tiles + COUNT_TILES - 1) / COUNT_TILES), dim3(256), 0, stream, reqs_d, 1u,
                            (const uint32_t *)w.counts);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(pixels, base + o_pix, px * 24, hipMemcpyDeviceToHost, stream));
-    if (hits) HIP_TRY(hipMemcpyAsync(hits, base + o_hits, px * 16, hipMemcpyDeviceToHost, stream));
-    HIP_TRY(hipMemcpyAsync(g_noalloc_counts, cnt_d, 40, hipMemcpyDeviceToHost, stream));
+    hipLaunchKernelGGL(k_deliver, dim3(seg_blocks + 1), dim3(DELIVER_THREADS), 0, stream, reqs_d, 1u, 0u,
+                       (const KSeg *)(base + o_segs), nseg, seg_blocks, (const unsigned long long *)cnt_d,
+                       (unsigned long long *)(g_noalloc_host_dev + ST_NOALLOC_COUNTS), 5u);
+    HIP_TRY(hipGetLastError());
+    if (!own_px) HIP_TRY(hipMemcpyAsync(pixels, base + o_pix, px * 24, hipMemcpyDeviceToHost, stream));
+    if (hits && !own_hits) HIP_TRY(hipMemcpyAsync(hits, base + o_hits, px * 16, hipMemcpyDeviceToHost, stream));
     HIP_TRY(hipStreamSynchronize(stream));
-    if (g_noalloc_counts[3])
+    const unsigned long long *counts_h = (const unsigned long long *)(g_noalloc_host + ST_NOALLOC_COUNTS);
+    if (counts_h[3])
         return set_err(ST_ERR_SCENE, "a traversal ran past its bound (fault bits 0x%llx): malformed BVH",
-                       g_noalloc_counts[3]);
+                       counts_h[3]);
     if (counts) {
         counts->primary = px;
-        counts->shadow = g_noalloc_counts[1];
-        counts->bounce = g_noalloc_counts[2];
+        counts->shadow = counts_h[1];
+        counts->bounce = counts_h[2];
     }
     return ST_OK;
 }
@@ -2496,22 +2676,23 @@ extern "C" int st_pick(StSceneHandle *scene, const StView *view, uint32_t n, con
     StHostView hv;
     if (st_view_prepare(scene->host, view, &hv)) return set_err(ST_ERR_ARG, "invalid view");
     const uint32_t P = scene->host->prim_count;
-    /* one upload block: request, scene descriptor, rects, points */
+    /* one upload block: request, scene descriptor, rects, points; behind it in
+       the page-locked staging the fault word and the picks, which the kernel
+       writes there */
     const size_t o_sc = round256(sizeof(KReq)), o_rect = o_sc + round256(sizeof(StDScene)),
-                 o_xy = o_rect + round256((P + 1) * 16ull), o_fault = o_xy + round256(n * 8ull),
-                 up = o_fault + 256;
-    if ((rc = arena_reserve(&g.main.work, up + round256(n * sizeof(StPick)) + 512)) || (rc = staging_reserve(&g.main, up))) {
+                 o_xy = o_rect + round256((P + 1) * 16ull), up = o_xy + round256(n * 8ull), o_fault = up,
+                 o_out = up + 256;
+    if ((rc = arena_reserve(&g.main.work, up + 512)) || (rc = staging_reserve(&g.main, o_out + n * sizeof(StPick)))) {
         st_view_release(&hv);
         return rc;
     }
     char *blk = (char *)arena_take(&g.main.work, up);
-    StPick *out_d = (StPick *)arena_take(&g.main.work, n * sizeof(StPick));
     KReq *rq = (KReq *)g.main.staging;
     memset(rq, 0, sizeof(KReq));
     rq->v = hv.dv;
     rq->v.rects = (const int32_t *)(blk + o_rect);
     StDScene dsc = scene->dev;
-    dsc.fault = (uint32_t *)(blk + o_fault);
+    dsc.fault = NULL;
     dsc.step_cap = g.step_cap;
     /* picking traces sequentially: its mesh traversals stop (a fault) at the
        bound no valid tree reaches, the largest mesh's node count */
@@ -2533,17 +2714,19 @@ extern "C" int st_pick(StSceneHandle *scene, const StView *view, uint32_t n, con
     memcpy(pk.rmi, rmi, sizeof rmi);
     pk.n = n;
     pk.xy = (const uint32_t *)(blk + o_xy);
-    pk.out = out_d;
+    pk.out = (StPick *)(g.main.staging_dev + o_out);
+    pk.fault = (uint32_t *)(g.main.staging_dev + o_fault);
     st_view_release(&hv);
     const uint32_t m_entries = scene->dev.mesh_stack_size > 1 ? scene->dev.mesh_stack_size : 1;
-    HIP_TRY(hipMemcpyAsync(blk, g.main.staging, up, hipMemcpyHostToDevice, g.main.stream));
+    hipLaunchKernelGGL(k_setup, dim3(setup_blocks(up)), dim3(SETUP_THREADS), 0, g.main.stream,
+                       (const uint4 *)g.main.staging_dev, (uint4 *)blk, (uint32_t)(up / 16),
+                       (unsigned long long *)NULL, 0u, (uint32_t *)NULL, 0u, (uint32_t *)NULL, (uint32_t *)NULL);
     hipLaunchKernelGGL(k_pick, dim3((n + 63) / 64), dim3(64), (size_t)64 * (1 + m_entries) * 4, g.main.stream,
                        (const StDScene *)(blk + o_sc), (const KReq *)blk, pk, m_entries);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(out, out_d, n * sizeof(StPick), hipMemcpyDeviceToHost, g.main.stream));
-    uint32_t fault = 0;
-    HIP_TRY(hipMemcpyAsync(&fault, blk + o_fault, 4, hipMemcpyDeviceToHost, g.main.stream));
     HIP_TRY(hipStreamSynchronize(g.main.stream));
+    const uint32_t fault = *(const uint32_t *)(g.main.staging + o_fault);
+    memcpy(out, g.main.staging + o_out, n * sizeof(StPick));
     if (fault) return set_err(ST_ERR_SCENE, "a traversal ran past its bound (fault bits 0x%x): malformed BVH", fault);
     return ST_OK;
 }
@@ -2568,8 +2751,10 @@ extern "C" int st_resolve_bgra8(const StFloatPixel *grid, uint32_t grid_w, uint3
     req_h->bgra = out_d;
     HIP_TRY(hipMemcpyAsync(grid_d, grid, gbytes, hipMemcpyHostToDevice, g.main.stream));
     HIP_TRY(hipMemcpyAsync(req_d, req_h, sizeof(KReq), hipMemcpyHostToDevice, g.main.stream));
-    hipLaunchKernelGGL(k_resolve, dim3((uint32_t)((opx + 255) / 256)), dim3(256), 0, g.main.stream, (const KReq *)req_d, 1u,
-                       (uint32_t)opx);
+    const uint32_t blocks = (uint32_t)((opx + RESOLVE_PIXELS - 1) / RESOLVE_PIXELS);
+    hipLaunchKernelGGL(k_deliver, dim3(blocks), dim3(DELIVER_THREADS), 0, g.main.stream, (const KReq *)req_d, 1u,
+                       blocks, (const KSeg *)NULL, 0u, 0u, (const unsigned long long *)NULL,
+                       (unsigned long long *)NULL, 0u);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(out, out_d, opx * 4, hipMemcpyDeviceToHost, g.main.stream));
     HIP_TRY(hipStreamSynchronize(g.main.stream));
@@ -2582,11 +2767,21 @@ extern "C" int st_host_alloc(size_t bytes, void **out) {
     int rc = ensure_init();
     if (rc) return rc;
     HIP_TRY(hipHostMalloc(out, bytes ? bytes : 1, hipHostMallocDefault));
+    void *d = NULL;
+    if (hipHostGetDevicePointer(&d, *out, 0) == hipSuccess && d == *out) {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        g_pinned[(uintptr_t)*out] = bytes ? bytes : 1;
+    }
     return ST_OK;
 }
 
 extern "C" void st_host_free(void *p) {
-    if (p) (void)hipHostFree(p);
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        g_pinned.erase((uintptr_t)p);
+    }
+    (void)hipHostFree(p);
 }
 
 /* ---- launch tuning ------------------------------------------------------ */

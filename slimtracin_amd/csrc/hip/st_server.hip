@@ -43,7 +43,7 @@ class PinnedPool {
   public:
     ~PinnedPool() {
         for (auto &kv : free_)
-            for (void *p : kv.second) (void)hipHostFree(p);
+            for (void *p : kv.second) st_host_free(p);
     }
     void *get(size_t bytes, size_t *cls_out) {
         size_t cls = 65536;
@@ -59,7 +59,7 @@ class PinnedPool {
             }
         }
         void *p = NULL;
-        if (hipHostMalloc(&p, cls, hipHostMallocDefault) != hipSuccess) return NULL;
+        if (st_host_alloc(cls, &p) != ST_OK) return NULL;
         return p;
     }
     void put(void *p, size_t cls) {

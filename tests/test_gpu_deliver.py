@@ -1,0 +1,92 @@
+"""GPU: outputs in page-locked memory (the device writes them itself at a
+launch's end) equal the same launch's outputs in pageable memory (copied):
+grids, hit records and window images of odd sizes, from one pixel up to more
+than one block's share, at every 4-byte offset, next to bytes that must stay
+as they are."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import slimtracin_amd as st
+from slimtracin_amd.scene import HIT_DTYPE, MODE_BEAUTY, MODE_NORMALS, PIXEL_DTYPE, make_view
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 1), (1, 7), (2, 1), (3, 3), (5, 2), (63, 17), (1023, 1), (1025, 3), (333, 41)]
+
+
+def _views():
+    return np.concatenate([make_view(width=w, height=h, mode=MODE_BEAUTY if i % 2 else MODE_NORMALS, depth=2,
+                                     position=(0.0, 7.0, -11.0), pitch=-0.2) for i, (w, h) in enumerate(SIZES)])
+
+
+@pytest.fixture(scope="module")
+def scene():
+    ds = st.DeviceScene(st.gen_implicit(3))
+    yield ds
+    ds.close()
+
+
+def _guarded(sizes, item, offset):
+    """Byte slices of one page-locked block at `offset` into a 16-byte grid, guard bytes between them."""
+    at, spans = offset, []
+    for n in sizes:
+        spans.append((at, at + n * item))
+        at += n * item + 12
+        at += (offset - at) % 16
+    block = st.pinned_empty(at + 64, np.uint8)
+    block[:] = 0xA5
+    return block, spans
+
+
+def _guards_stand(block, spans):
+    outside = np.ones(len(block), bool)
+    for a, b in spans:
+        outside[a:b] = False
+    return bool((block[outside] == 0xA5).all())
+
+
+@pytest.mark.parametrize("offset", [0, 4, 8, 12])
+def test_window_images(scene, offset):
+    views = _views()
+    want, _ = st.render_batch_bgra8([scene] * len(views), views)
+    block, spans = _guarded([w * h for w, h in SIZES], 4, offset)
+    outs = [block[a:b].view(np.uint32) for a, b in spans]
+    got, counts = st.render_batch_bgra8([scene] * len(views), views, outs=outs)
+    for g, w in zip(got, want):
+        assert (g == w).all()
+    assert _guards_stand(block, spans)
+    assert [c.primary for c in counts] == [(w + 1) * (h + 1) for w, h in SIZES]
+
+
+@pytest.mark.parametrize("offset", [0, 8])
+@pytest.mark.parametrize("call", ["batch", "plain", "noalloc"])
+def test_grids_and_hits(scene, offset, call):
+    views = _views()
+    n = len(views)
+    grid = [(w + 1) * (h + 1) for w, h in SIZES]
+    want_p, want_h, want_c = st.render_batch([scene] * n, views, hits=True)
+    pb, ps = _guarded(grid, PIXEL_DTYPE.itemsize, offset)
+    hb, hs = _guarded(grid, HIT_DTYPE.itemsize, offset)
+    pix = [pb[a:b].view(PIXEL_DTYPE) for a, b in ps]
+    hits = [hb[a:b].view(HIT_DTYPE) for a, b in hs]
+    counts = (st.RayCounts * n)()
+    L = st.lib()
+    if call == "batch":
+        handles = (C.c_void_p * n)(*[scene.handle] * n)
+        rc = L.st_render_batch(handles, views.ctypes.data_as(C.c_void_p), C.c_uint32(n),
+                               (C.c_void_p * n)(*[p.ctypes.data for p in pix]),
+                               (C.c_void_p * n)(*[h.ctypes.data for h in hits]), counts, C.c_uint32(1))
+        assert rc == 0
+    else:
+        fn = L.st_render if call == "plain" else L.st_render_noalloc
+        for i in range(n):
+            assert fn(scene.handle, views[i:i + 1].ctypes.data_as(C.c_void_p), C.c_void_p(pix[i].ctypes.data),
+                      C.c_void_p(hits[i].ctypes.data), C.byref(counts[i])) == 0
+    for i in range(n):
+        assert pix[i].tobytes() == want_p[i].tobytes() and hits[i].tobytes() == want_h[i].tobytes()
+        assert (counts[i].shadow, counts[i].bounce) == (want_c[i].shadow, want_c[i].bounce)
+    assert _guards_stand(pb, ps) and _guards_stand(hb, hs)
