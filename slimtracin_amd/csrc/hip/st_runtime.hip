@@ -65,6 +65,7 @@
 #include "slimtracin.h"
 #include "st_internal.h"
 #include "st_sort.h"
+#include "st_copy.h"
 
 #define WAVES_PER_BLOCK 4
 #define BLOCK_THREADS (64 * WAVES_PER_BLOCK)
@@ -1213,6 +1214,7 @@ struct LaunchCtx {
     Arena work;            /* per-launch device buffers (grow-only) */
     char *staging;         /* pinned host staging: uploads, then the ray-count readback */
     char *staging_dev;     /* the same memory at the device's address */
+    CopyRing ring;         /* for large copies of pageable memory */
     size_t staging_cap;
     uint32_t *tile_cost;   /* [tile_cap] each tile's time in the last primary stage */
     uint32_t *tile_order;  /* [tile_cap] the primary stage's claim order (order_tiles) */
@@ -1295,6 +1297,7 @@ static void ctx_release(LaunchCtx *c) {
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
     if (c->work.base) (void)hipFree(c->work.base);
     if (c->staging) (void)hipHostFree(c->staging);
+    copy_ring_release(&c->ring);
     if (c->tile_cost) (void)hipFree(c->tile_cost);
     if (c->cost_sum) (void)hipFree(c->cost_sum);
     if (c->tile_counter) (void)hipFree(c->tile_counter);
@@ -1442,7 +1445,7 @@ extern "C" int st_scene_create_ex(const void *blob, size_t size, uint32_t flags,
     if ((flags & ST_SCENE_MESH_LBVH) && (flags & ST_SCENE_MESH_BINNED))
         return set_err(ST_ERR_ARG, "ST_SCENE_MESH_LBVH and ST_SCENE_MESH_BINNED together");
     const char *why = NULL;
-    uint32_t builder = (flags & ST_SCENE_MESH_LBVH)     ? ST_MESH_BUILD_DEVICE
+    uint32_t builder = (flags & ST_SCENE_MESH_LBVH)     ? ST_MESH_BUILD_DEVICE_UNCHECKED
                        : (flags & ST_SCENE_MESH_BINNED) ? ST_MESH_BUILD_BINNED
                                                         : ST_MESH_BUILD_SAH;
     StScene *sc = st_scene_from_blob_ex(blob, size, builder, &why);
@@ -1464,6 +1467,7 @@ extern "C" int st_scene_create(const void *blob, size_t size, StSceneHandle **ou
 /* Device LBVH builds of the meshes the host left unbuilt: geometry goes to a
    scratch buffer, nodes and triangle records straight into the scene's
    allocation, then the heights come back for the traversal stack size. */
+#define MESH_SCRATCH_SHARED (256ull << 20)
 static int build_device_meshes(StSceneHandle *h) {
     StScene *sc = h->host;
     size_t geom = 0, work = 0, sort_bytes = 0;
@@ -1482,9 +1486,17 @@ static int build_device_meshes(StSceneHandle *h) {
         any = 1;
     }
     if (!any) return ST_OK;
-    char *buf = NULL;
-    hipError_t e = hipMalloc(&buf, geom + work + 256);
-    if (e != hipSuccess) return set_err(ST_ERR_MEMORY, "hipMalloc(%zu) for mesh builds failed", geom + work);
+    /* a build's scratch: the main context's buffer up to a size that its
+       launches need anyway, else memory of its own (an allocation and its
+       release take 0.4 ms) */
+    char *own = NULL, *buf = NULL;
+    if (geom + work <= MESH_SCRATCH_SHARED && arena_reserve(&g.main.work, geom + work + 512) == ST_OK) {
+        buf = (char *)arena_take(&g.main.work, geom + work + 256);
+    } else {
+        hipError_t e = hipMalloc(&own, geom + work + 256);
+        if (e != hipSuccess) return set_err(ST_ERR_MEMORY, "hipMalloc(%zu) for mesh builds failed", geom + work);
+        buf = own;
+    }
     uint32_t *height_d = (uint32_t *)(buf + geom + work);
     int rc = ST_OK;
     uint32_t max_height = 0;
@@ -1496,22 +1508,35 @@ static int build_device_meshes(StSceneHandle *h) {
         StMeshGeomDev in;
         memset(&in, 0, sizeof in);
         in.T = q->triangle_count;
-        struct { const void *src; size_t bytes; const void **dst; } up[6] = {
-            {s->pos, 12ull * q->vertex_count, (const void **)&in.pos},
-            {s->pidx, 12ull * q->triangle_count, (const void **)&in.pidx},
-            {q->normals_count ? s->nrm : NULL, 12ull * q->normals_count, (const void **)&in.nrm},
-            {q->normals_count ? s->nidx : NULL, 12ull * q->triangle_count, (const void **)&in.nidx},
-            {q->uvs_count ? s->uvs : NULL, 8ull * q->uvs_count, (const void **)&in.uvs},
-            {q->uvs_count ? s->uidx : NULL, 12ull * q->triangle_count, (const void **)&in.uidx},
+        /* indices are checked on their way (the scene was parsed without) */
+        struct { const void *src; size_t bytes; const void **dst; uint32_t limit; } up[6] = {
+            {s->pos, 12ull * q->vertex_count, (const void **)&in.pos, 0},
+            {s->pidx, 12ull * q->triangle_count, (const void **)&in.pidx, q->vertex_count},
+            {q->normals_count ? s->nrm : NULL, 12ull * q->normals_count, (const void **)&in.nrm, 0},
+            {q->normals_count ? s->nidx : NULL, 12ull * q->triangle_count, (const void **)&in.nidx, q->normals_count},
+            {q->uvs_count ? s->uvs : NULL, 8ull * q->uvs_count, (const void **)&in.uvs, 0},
+            {q->uvs_count ? s->uidx : NULL, 12ull * q->triangle_count, (const void **)&in.uidx, q->uvs_count},
         };
-        for (int k = 0; k < 6 && !rc; k++) {
+        std::vector<CopySpan> spans;
+        for (int k = 0; k < 6; k++) {
             if (!up[k].src || !up[k].bytes) continue;
-            if (hipMemcpyAsync(p, up[k].src, up[k].bytes, hipMemcpyHostToDevice, g.main.stream) != hipSuccess)
-                rc = set_err(ST_ERR_HIP, "mesh geometry upload failed");
+            spans.push_back({p, (char *)up[k].src, up[k].bytes, up[k].limit});
             *up[k].dst = p;
             p += round256(up[k].bytes);
         }
-        if (rc) break;
+        bool in_range = false;
+        if (q->vertex_count == 0) {
+            rc = set_err(ST_ERR_SCENE, "invalid scene: mesh index out of range");
+            break;
+        }
+        if (copy_pageable(g.main.stream, &g.main.ring, spans, false, &in_range) != hipSuccess) {
+            rc = set_err(ST_ERR_HIP, "mesh geometry upload failed");
+            break;
+        }
+        if (!in_range) {
+            rc = set_err(ST_ERR_SCENE, "invalid scene: mesh index out of range");
+            break;
+        }
         const StDMesh &dm = sc->meshes[m];
         uint32_t *nodes = (uint32_t *)h->dev.mesh_nodes + 8ull * dm.node_offset;
         StDTriHot *hot = (StDTriHot *)h->dev.tri_hot + dm.tri_offset;
@@ -1535,7 +1560,7 @@ static int build_device_meshes(StSceneHandle *h) {
         memset(sc->deferred + m, 0, sizeof(StMeshPart));
     }
     (void)hipStreamSynchronize(g.main.stream);
-    (void)hipFree(buf);
+    if (own) (void)hipFree(own);
     if (rc) return rc;
     sc->max_mesh_height = max_height;
     sc->mesh_stack_size = (uint8_t)(max_height + 2); /* core/init.h:523-527 */
@@ -1624,8 +1649,10 @@ extern "C" int st_scene_upload(StSceneHandle *h) {
         {o_mips, sc->mips, sc->mip_total * sizeof(StDMip)},
         {o_texels, sc->texels, sc->texel_bytes},
     };
+    std::vector<CopySpan> spans;
     for (size_t i = 0; i < sizeof parts / sizeof parts[0]; i++)
-        if (parts[i].bytes) HIP_TRY(hipMemcpy(b + parts[i].off, parts[i].src, parts[i].bytes, hipMemcpyHostToDevice));
+        if (parts[i].bytes) spans.push_back({b + parts[i].off, (char *)parts[i].src, parts[i].bytes, 0});
+    HIP_TRY(copy_pageable(g.main.stream, &g.main.ring, spans, false));
     if (sc->mesh_count) {
         float *ma = (float *)malloc(24ull * sc->mesh_count);
         for (uint32_t m = 0; m < sc->mesh_count; m++) {
@@ -2275,17 +2302,18 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
                        (const unsigned long long *)cnt_d, (unsigned long long *)(c->staging_dev + o_readback),
                        3 * n + 2);
     HIP_TRY(hipGetLastError());
+    std::vector<CopySpan> spans;
     for (uint32_t i = 0; i < n; i++) {
         size_t px = (size_t)hv[i].dv.width1 * hv[i].dv.height1;
         if (pixels_host && pixels_host[i] && !own_px[i])
-            HIP_TRY(hipMemcpyAsync(pixels_host[i], reqs_h[i].v.pixels, px * 24, hipMemcpyDeviceToHost, c->stream));
+            spans.push_back({(char *)reqs_h[i].v.pixels, (char *)pixels_host[i], px * 24, 0});
         if (hits_host && hits_host[i] && want_hits && !own_hits[i])
-            HIP_TRY(hipMemcpyAsync(hits_host[i], reqs_h[i].v.hits, px * 16, hipMemcpyDeviceToHost, c->stream));
+            spans.push_back({(char *)reqs_h[i].v.hits, (char *)hits_host[i], px * 16, 0});
         if (reqs_h[i].bgra && !own_bgra[i])
-            HIP_TRY(hipMemcpyAsync(bgra_host[i], reqs_h[i].bgra,
-                                   (size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4, hipMemcpyDeviceToHost,
-                                   c->stream));
+            spans.push_back({(char *)reqs_h[i].bgra, (char *)bgra_host[i],
+                             (size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4, 0});
     }
+    if (!spans.empty()) HIP_TRY(copy_pageable(c->stream, &c->ring, spans, true));
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->last_redo = (uint32_t)cnt_h[3 * (size_t)n + 1];
     if (cnt_h[3 * (size_t)n])

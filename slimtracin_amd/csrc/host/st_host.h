@@ -105,6 +105,8 @@ typedef struct StSceneParts {
 #define ST_MESH_BUILD_SAH 0u
 #define ST_MESH_BUILD_DEVICE 1u
 #define ST_MESH_BUILD_BINNED 2u
+/* ST_MESH_BUILD_DEVICE with the caller checking the meshes' indices */
+#define ST_MESH_BUILD_DEVICE_UNCHECKED 3u
 
 /* Validate the parts and build the device-ready scene. Returns NULL on
    malformed input; *err (if given) receives a short reason. */

@@ -208,7 +208,7 @@ StScene *st_scene_from_parts(const StSceneParts *pp, const char **err) {
         } else if (!s->pos || !s->pidx) {
             FAIL("mesh without geometry");
         }
-        if (s->pidx)
+        if (s->pidx && (q->prebuilt || pp->mesh_builder != ST_MESH_BUILD_DEVICE_UNCHECKED))
             for (uint64_t t = 0; t < 3ull * q->triangle_count; t++)
                 if (s->pidx[t] >= q->vertex_count || (s->nidx && s->nidx[t] >= q->normals_count) ||
                     (s->uidx && s->uidx[t] >= q->uvs_count))
@@ -232,9 +232,11 @@ StScene *st_scene_from_parts(const StSceneParts *pp, const char **err) {
     if (!sc->mesh_on_device || !sc->deferred) FAIL("out of host memory");
     /* host copies of the mesh records only when some mesh is built or
        loaded on the host; device-built meshes never have one */
+    const int on_device = pp->mesh_builder == ST_MESH_BUILD_DEVICE ||
+                          pp->mesh_builder == ST_MESH_BUILD_DEVICE_UNCHECKED;
     sc->mesh_host_data = pp->mesh_count ? 0u : 1u;
     for (uint32_t m = 0; m < pp->mesh_count; m++)
-        if (pp->meshes[m].rec.prebuilt || pp->mesh_builder != ST_MESH_BUILD_DEVICE) sc->mesh_host_data = 1;
+        if (pp->meshes[m].rec.prebuilt || !on_device) sc->mesh_host_data = 1;
     sc->mesh_nodes = (StBVHNodeRec *)calloc(sc->mesh_host_data ? node_total + 1 : 1, sizeof(StBVHNodeRec));
     sc->tri_hot = (StDTriHot *)calloc(sc->mesh_host_data ? tri_total + 1 : 1, sizeof(StDTriHot));
     sc->tri_cold = (StDTriCold *)calloc(sc->mesh_host_data ? tri_total + 1 : 1, sizeof(StDTriCold));
@@ -244,7 +246,7 @@ StScene *st_scene_from_parts(const StSceneParts *pp, const char **err) {
         const StMeshRec *q = &s->rec;
         StDMesh *dm = sc->meshes + m;
         uint32_t height = 0, count = 0;
-        if (!q->prebuilt && pp->mesh_builder == ST_MESH_BUILD_DEVICE) {
+        if (!q->prebuilt && on_device) {
             sc->mesh_on_device[m] = 1;
             sc->deferred[m] = *s;
             dm->height = 0;
