@@ -116,6 +116,9 @@ struct KReq {
     uint32_t out_block;    /* first block of the display resolve for this request (k_deliver) */
     uint32_t count_block;  /* first block of k_counts for this request */
     uint32_t *bgra;        /* window image (width1-1)*(height1-1), or NULL */
+    /* where the device itself writes the traced grid and the hit records
+       (page-locked host memory), or NULL */
+    char *px_out, *hits_out;
     uint64_t pad2;
     /* device SSB pass (k_ssb) when device_ssb: camera rotation_matrix_inverted
        (rows X, Y, Z) and focal length; ssb_raw / ssb_flags optionally receive
@@ -416,6 +419,168 @@ __device__ static inline __attribute__((always_inline)) void primary_tile(const 
     primary_pixel<false>(sc, v, tile * 64u + lane, x, y, valid, box, stk, w);
 }
 
+/* Display resolve of one window pixel (drawViewportToWindowContent,
+   viewport/viewport.h:12-66, QCAA branch): the 4 traced corners are averaged
+   as (TL.c*TL.o + (TR.c*TR.o + (BL.c*BL.o + BR.c*BR.o))) * 0.25 and each
+   channel is (u8)sqrt(c), 255 above 255^2. (u8) of the double square root is
+   floor(sqrt(c)): computed exactly in integers from the correctly rounded
+   fp32 root (squares up to 255^2 are exact in fp32). Background (all four
+   depths infinite) is (0,0,0,255); alpha is 255 everywhere; NaN or negative
+   channels give 0. Bytes B, G, R, A. */
+__device__ static inline uint32_t resolve_channel(float c) {
+    if (c > 65025.0f) return 255u;
+    if (!(c >= 0.0f)) return 0u;
+    uint32_t s = (uint32_t)sqrtf(c);
+    if (s > 255u) s = 255u;
+    while (s < 255u && (float)((s + 1u) * (s + 1u)) <= c) s++;
+    while (s > 0u && (float)(s * s) > c) s--;
+    return s;
+}
+
+/* Window pixels [at, at + n) of a request's image, n at most 4: neighbours
+   share their corners. */
+__device__ static inline void resolve_pixels(const KReq &r, uint32_t at, uint32_t n) {
+    const uint32_t w1 = r.v.width1, w = w1 - 1u;
+    const char *base = static_cast<const char *>(r.v.pixels);
+    uint32_t y = at / w, x = at - y * w;
+    uint32_t out[4];
+    float right[2][4];
+    bool right_background = false;
+    for (uint32_t k = 0; k < n; k++) {
+        const bool fresh = k == 0 || x == 0;   /* the left corners are not the last pixel's right ones */
+        float c[4][4];
+        bool background = true;
+        for (int j = 0; j < 4; j++) {
+            /* TL, TR, BL, BR */
+            if (!(j & 1) && !fresh) {
+                for (int e = 0; e < 4; e++) c[j][e] = right[j >> 1][e];
+                continue;
+            }
+            /* 24-byte records are 8-byte aligned: three 8-byte loads */
+            const char *p = base + 24 * ((size_t)(y + (uint32_t)(j >> 1)) * w1 + x + (uint32_t)(j & 1));
+            const float2 rg = *reinterpret_cast<const float2 *>(p);
+            const float2 bo = *reinterpret_cast<const float2 *>(p + 8);
+            const double d = *reinterpret_cast<const double *>(p + 16);
+            c[j][0] = rg.x; c[j][1] = rg.y; c[j][2] = bo.x; c[j][3] = bo.y;
+            const bool far = d == (double)INFINITY;
+            if (j & 1) {
+                for (int e = 0; e < 4; e++) right[j >> 1][e] = c[j][e];
+                background = background && far;
+            } else {
+                right_background = j == 0 ? far : right_background && far;
+            }
+        }
+        /* right_background: so far the left corners' (the last pixel's right ones) */
+        const bool all = background && right_background;
+        right_background = background;
+        uint32_t px = 0xFF000000u;
+        if (!all) {
+            uint32_t ch[3];
+            for (int e = 0; e < 3; e++) {
+                float acc = c[3][e] * c[3][3];
+                acc = c[2][e] * c[2][3] + acc;
+                acc = c[1][e] * c[1][3] + acc;
+                acc = c[0][e] * c[0][3] + acc;
+                ch[e] = resolve_channel(acc * 0.25f);
+            }
+            px |= ch[2] | (ch[1] << 8) | (ch[0] << 16);
+        }
+        out[k] = px;
+        if (++x == w) { x = 0; y++; }
+    }
+    uint32_t *o = r.bgra + at;
+    if (n == 4u && ((uintptr_t)o & 15u) == 0) {
+        *reinterpret_cast<uint4 *>(o) = make_uint4(out[0], out[1], out[2], out[3]);
+    } else {
+        for (uint32_t k = 0; k < n; k++) o[k] = out[k];
+    }
+}
+
+/* What a launch hands over, in one launch at its end: window images (the
+   display resolve, straight to where they go), traced grids and hit records
+   (16 KB of a segment per block), and the ray counts. Destinations are
+   page-locked host memory that the device writes over the link, or device
+   buffers that are copied on from there. Bound by the link (50 of its 57 GB/s):
+   160 window images, 189 MB, take 3.8 ms; resolved into device memory
+   (0.7 ms) and copied by a call each they took 7. Plain requests of a mixed
+   launch go out earlier (KEarly). */
+#define DELIVER_THREADS 256u
+#define RESOLVE_PIXELS (4u * DELIVER_THREADS)   /* per block */
+#define SEG_CHUNK 16384u
+struct KSeg {
+    const char *src;
+    char *dst;
+    uint64_t bytes;        /* a multiple of 4, as are both addresses */
+    uint32_t first_block;
+    uint32_t pad;
+};
+__device__ static inline void copy_segment(const KSeg &g, uint32_t chunk) {
+    const uint64_t at = (uint64_t)chunk * SEG_CHUNK;
+    const uint32_t n = (uint32_t)min((uint64_t)SEG_CHUNK, g.bytes - at);
+    const char *src = g.src + at;
+    char *dst = g.dst + at;
+    if ((((uintptr_t)src | (uintptr_t)dst) & 15u) == 0) {
+        for (uint32_t i = threadIdx.x * 16u; i + 16u <= n; i += DELIVER_THREADS * 16u)
+            *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(src + i);
+        const uint32_t tail = n & ~15u;
+        for (uint32_t i = tail + threadIdx.x * 4u; i < n; i += DELIVER_THREADS * 4u)
+            *reinterpret_cast<uint32_t *>(dst + i) = *reinterpret_cast<const uint32_t *>(src + i);
+    } else {
+        for (uint32_t i = threadIdx.x * 4u; i < n; i += DELIVER_THREADS * 4u)
+            *reinterpret_cast<uint32_t *>(dst + i) = *reinterpret_cast<const uint32_t *>(src + i);
+    }
+}
+/* Share `b` of a launch's delivery: resolve shares first, then segments'. */
+__device__ static inline void deliver_share(const KReq *reqs, uint32_t nreq, uint32_t resolve_blocks,
+                                            const KSeg *segs, uint32_t nseg, uint32_t b) {
+    uint32_t lo = 0;
+    if (b < resolve_blocks) {
+        uint32_t hi = nreq - 1;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1) >> 1;
+            if (reqs[mid].out_block <= b) lo = mid; else hi = mid - 1;
+        }
+        const KReq &r = reqs[lo];
+        const uint32_t at = (b - r.out_block) * RESOLVE_PIXELS + 4u * threadIdx.x;
+        const uint32_t total = r.bgra ? (r.v.width1 - 1u) * (r.v.height1 - 1u) : 0u;
+        if (at < total) resolve_pixels(r, at, min(4u, total - at));
+    } else {
+        b -= resolve_blocks;
+        uint32_t hi = nseg - 1;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1) >> 1;
+            if (segs[mid].first_block <= b) lo = mid; else hi = mid - 1;
+        }
+        copy_segment(segs[lo], b - segs[lo].first_block);
+    }
+}
+
+/* Delivery during the primary stage. A launch whose requests include both
+   plain ones (no bounce stage: only the primary stage, and now and then the
+   redo stage, writes their pixels) and others runs its primary stage in two
+   kernels, the plain requests' tiles first, and the second kernel's first
+   EARLY_BLOCKS blocks write the plain requests' outputs over the link before
+   they take tiles: the stage is bound by issue slots, the delivery by the
+   link. Pixels that the redo stage changes afterwards are written again by
+   k_deliver. 160 requests with 142 MB of plain window images: 15.25 -> 13.6
+   ms (the primary stage 8.2 -> 9.2, the delivery after it 3.8 -> 0.87);
+   with 32, 128 or 256 such blocks 17.0, 13.8, 14.4. One kernel whose waves
+   count themselves out of the plain tiles, without a drain between, took
+   13.7. */
+#define EARLY_BLOCKS 64u
+#define EARLY_CLAIMS 512u              /* the second kernel's counters, after the first's */
+/* Plain outputs and other requests' pixels below which one kernel is the
+   quicker: the drain between the two costs about 0.2 ms. 20 MB (20 requests):
+   2.97 ms in one kernel, 3.17 in two; 45 MB (160 of up to 700 pixels a side):
+   5.78, 5.76. */
+#define EARLY_MIN_BYTES (48ull << 20)
+#define EARLY_MIN_PIXELS (1u << 21)
+struct KEarly {
+    const KSeg *segs;
+    uint32_t nreq, nseg;               /* the plain requests and their segments: the first of the launch's */
+    uint32_t resolve_blocks, shares;   /* shares 0: nothing to deliver */
+};
+
 /* Traversal stacks live in LDS, one column per lane (no bank conflicts):
    [wave][entry][lane]. */
 #define ST_LDS_STACKS(scene_entries, mesh_entries)                                                              \
@@ -458,7 +623,10 @@ __device__ static inline __attribute__((always_inline)) void
 primary_stage(const StDScene *__restrict__ scenes, const KReq *__restrict__ reqs, uint32_t nreq, uint32_t total_tiles,
               uint32_t *tile_counter, uint32_t persistent, uint32_t xcd_blocks, uint32_t scene_entries,
               uint32_t mesh_entries, const KWave &w, const uint32_t *__restrict__ tile_order,
-              uint32_t *__restrict__ tile_cost) {
+              uint32_t *__restrict__ tile_cost, const KEarly &early) {
+    if (blockIdx.x < EARLY_BLOCKS)
+        for (uint32_t s = blockIdx.x; s < early.shares; s += min(gridDim.x, EARLY_BLOCKS))
+            deliver_share(reqs, early.nreq, early.resolve_blocks, early.segs, early.nseg, s);
     ST_LDS_STACKS(scene_entries, mesh_entries);
     const DStacks stk = {scene_stack, mesh_stack, nullptr};
     /* One call site, so primary_tile is inlined once. Persistent (1): waves
@@ -497,7 +665,8 @@ primary_stage(const StDScene *__restrict__ scenes, const KReq *__restrict__ reqs
 #define K_PRIMARY_ARGS                                                                                                \
     const StDScene *__restrict__ scenes, const KReq *__restrict__ reqs, uint32_t nreq, uint32_t total_tiles,         \
         uint32_t *tile_counter, uint32_t persistent, uint32_t xcd_blocks, uint32_t scene_entries,                     \
-        uint32_t mesh_entries, KWave w, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ tile_cost
+        uint32_t mesh_entries, KWave w, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ tile_cost,    \
+        KEarly early
 /* The primary stage at the occupancy its registers allow (3 waves per
    SIMD), and held to 4 waves per SIMD (128 registers, a few values in
    scratch) for launches whose traversal stacks leave LDS for 4 waves
@@ -505,11 +674,11 @@ primary_stage(const StDScene *__restrict__ scenes, const KReq *__restrict__ reqs
    primary stage took 30.0 ms at 4 waves against 34.2 ms at 3. */
 __global__ void __launch_bounds__(BLOCK_THREADS) K_PRIMARY_ATTR k_primary(K_PRIMARY_ARGS) {
     primary_stage(scenes, reqs, nreq, total_tiles, tile_counter, persistent, xcd_blocks, scene_entries, mesh_entries,
-                  w, tile_order, tile_cost);
+                  w, tile_order, tile_cost, early);
 }
 __global__ void __launch_bounds__(BLOCK_THREADS) __attribute__((amdgpu_waves_per_eu(4))) k_primary4(K_PRIMARY_ARGS) {
     primary_stage(scenes, reqs, nreq, total_tiles, tile_counter, persistent, xcd_blocks, scene_entries, mesh_entries,
-                  w, tile_order, tile_cost);
+                  w, tile_order, tile_cost, early);
 }
 
 /* Redo stage: the pixels whose traversal gave up in the main stages, each
@@ -1008,139 +1177,54 @@ __global__ void __launch_bounds__(64) k_pick(const StDScene *__restrict__ scenes
     stg2(o, 2, __float_as_uint(out[4]), __float_as_uint(out[5]));
 }
 
-/* Display resolve of one window pixel (drawViewportToWindowContent,
-   viewport/viewport.h:12-66, QCAA branch): the 4 traced corners are averaged
-   as (TL.c*TL.o + (TR.c*TR.o + (BL.c*BL.o + BR.c*BR.o))) * 0.25 and each
-   channel is (u8)sqrt(c), 255 above 255^2. (u8) of the double square root is
-   floor(sqrt(c)): computed exactly in integers from the correctly rounded
-   fp32 root (squares up to 255^2 are exact in fp32). Background (all four
-   depths infinite) is (0,0,0,255); alpha is 255 everywhere; NaN or negative
-   channels give 0. Bytes B, G, R, A. */
-__device__ static inline uint32_t resolve_channel(float c) {
-    if (c > 65025.0f) return 255u;
-    if (!(c >= 0.0f)) return 0u;
-    uint32_t s = (uint32_t)sqrtf(c);
-    if (s > 255u) s = 255u;
-    while (s < 255u && (float)((s + 1u) * (s + 1u)) <= c) s++;
-    while (s > 0u && (float)(s * s) > c) s--;
-    return s;
-}
-
-/* Window pixels [at, at + n) of a request's image, n at most 4: neighbours
-   share their corners. */
-__device__ static inline void resolve_pixels(const KReq &r, uint32_t at, uint32_t n) {
-    const uint32_t w1 = r.v.width1, w = w1 - 1u;
-    const char *base = static_cast<const char *>(r.v.pixels);
-    uint32_t y = at / w, x = at - y * w;
-    uint32_t out[4];
-    float right[2][4];
-    bool right_background = false;
-    for (uint32_t k = 0; k < n; k++) {
-        const bool fresh = k == 0 || x == 0;   /* the left corners are not the last pixel's right ones */
-        float c[4][4];
-        bool background = true;
-        for (int j = 0; j < 4; j++) {
-            /* TL, TR, BL, BR */
-            if (!(j & 1) && !fresh) {
-                for (int e = 0; e < 4; e++) c[j][e] = right[j >> 1][e];
-                continue;
-            }
-            /* 24-byte records are 8-byte aligned: three 8-byte loads */
-            const char *p = base + 24 * ((size_t)(y + (uint32_t)(j >> 1)) * w1 + x + (uint32_t)(j & 1));
-            const float2 rg = *reinterpret_cast<const float2 *>(p);
-            const float2 bo = *reinterpret_cast<const float2 *>(p + 8);
-            const double d = *reinterpret_cast<const double *>(p + 16);
-            c[j][0] = rg.x; c[j][1] = rg.y; c[j][2] = bo.x; c[j][3] = bo.y;
-            const bool far = d == (double)INFINITY;
-            if (j & 1) {
-                for (int e = 0; e < 4; e++) right[j >> 1][e] = c[j][e];
-                background = background && far;
-            } else {
-                right_background = j == 0 ? far : right_background && far;
-            }
+/* One redone pixel of a request whose outputs went out before the redo
+   stage: its grid and hit records and the window pixels it is a corner of. */
+__device__ static inline void deliver_again(const KReq &r, uint32_t slot) {
+    uint32_t x, y;
+    if (!tile_pixel(r.v, slot >> 6, slot & 63u, x, y)) return;
+    const size_t pix = (size_t)y * r.v.width1 + x;
+    if (r.px_out)
+        for (uint32_t k = 0; k < 6; k++)
+            reinterpret_cast<uint32_t *>(r.px_out)[pix * 6 + k] = reinterpret_cast<const uint32_t *>(r.v.pixels)[pix * 6 + k];
+    if (r.hits_out)
+        for (uint32_t k = 0; k < 4; k++)
+            reinterpret_cast<uint32_t *>(r.hits_out)[pix * 4 + k] = reinterpret_cast<const uint32_t *>(r.v.hits)[pix * 4 + k];
+    if (r.bgra) {
+        const uint32_t w = r.v.width1 - 1u, h = r.v.height1 - 1u;
+        for (uint32_t j = 0; j < 4; j++) {
+            const uint32_t wx = x - (j & 1u), wy = y - (j >> 1);
+            if (wx < w && wy < h) resolve_pixels(r, wy * w + wx, 1u);
         }
-        /* right_background: so far the left corners' (the last pixel's right ones) */
-        const bool all = background && right_background;
-        right_background = background;
-        uint32_t px = 0xFF000000u;
-        if (!all) {
-            uint32_t ch[3];
-            for (int e = 0; e < 3; e++) {
-                float acc = c[3][e] * c[3][3];
-                acc = c[2][e] * c[2][3] + acc;
-                acc = c[1][e] * c[1][3] + acc;
-                acc = c[0][e] * c[0][3] + acc;
-                ch[e] = resolve_channel(acc * 0.25f);
-            }
-            px |= ch[2] | (ch[1] << 8) | (ch[0] << 16);
-        }
-        out[k] = px;
-        if (++x == w) { x = 0; y++; }
-    }
-    uint32_t *o = r.bgra + at;
-    if (n == 4u && ((uintptr_t)o & 15u) == 0) {
-        *reinterpret_cast<uint4 *>(o) = make_uint4(out[0], out[1], out[2], out[3]);
-    } else {
-        for (uint32_t k = 0; k < n; k++) o[k] = out[k];
     }
 }
 
-/* What a launch hands over, in one launch at its end: window images (the
-   display resolve, straight to where they go), traced grids and hit records
-   (16 KB of a segment per block), and the ray counts. Destinations are
-   page-locked host memory that the device writes over the link, or device
-   buffers that are copied on from there. Bound by the link (50 of its 57 GB/s):
-   160 window images, 189 MB, take 3.8 ms; resolved into device memory
-   (0.7 ms) and copied by a call each they took 7. */
-#define DELIVER_THREADS 256u
-#define RESOLVE_PIXELS (4u * DELIVER_THREADS)   /* per block */
-#define SEG_CHUNK 16384u
-struct KSeg {
-    const char *src;
-    char *dst;
-    uint64_t bytes;        /* a multiple of 4, as are both addresses */
-    uint32_t first_block;
-    uint32_t pad;
+/* `shares` shares from first.resolve on (window images) and from first.seg on
+   (segments), the counts, and the redone pixels of the requests that went out
+   before (early_reqs, the launch's first). */
+struct KDeliver {
+    const KSeg *segs;
+    uint32_t nseg;
+    uint32_t resolve_first, resolve_blocks;   /* shares already out, and of all requests */
+    uint32_t seg_first, seg_blocks;
+    uint32_t early_reqs, again_blocks;
+    const uint32_t *redo_ctr, *redo_q;
 };
-__device__ static inline void copy_segment(const KSeg &g, uint32_t chunk) {
-    const uint64_t at = (uint64_t)chunk * SEG_CHUNK;
-    const uint32_t n = (uint32_t)min((uint64_t)SEG_CHUNK, g.bytes - at);
-    const char *src = g.src + at;
-    char *dst = g.dst + at;
-    if ((((uintptr_t)src | (uintptr_t)dst) & 15u) == 0) {
-        for (uint32_t i = threadIdx.x * 16u; i + 16u <= n; i += DELIVER_THREADS * 16u)
-            *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(src + i);
-        const uint32_t tail = n & ~15u;
-        for (uint32_t i = tail + threadIdx.x * 4u; i < n; i += DELIVER_THREADS * 4u)
-            *reinterpret_cast<uint32_t *>(dst + i) = *reinterpret_cast<const uint32_t *>(src + i);
-    } else {
-        for (uint32_t i = threadIdx.x * 4u; i < n; i += DELIVER_THREADS * 4u)
-            *reinterpret_cast<uint32_t *>(dst + i) = *reinterpret_cast<const uint32_t *>(src + i);
-    }
-}
-__global__ void __launch_bounds__(DELIVER_THREADS) k_deliver(const KReq *__restrict__ reqs, uint32_t nreq,
-                                                             uint32_t resolve_blocks, const KSeg *__restrict__ segs,
-                                                             uint32_t nseg, uint32_t seg_blocks,
+__global__ void __launch_bounds__(DELIVER_THREADS) k_deliver(const KReq *__restrict__ reqs, uint32_t nreq, KDeliver d,
                                                              const unsigned long long *counts,
                                                              unsigned long long *counts_out, uint32_t ncounts) {
+    const uint32_t resolves = d.resolve_blocks - d.resolve_first, segs = d.seg_blocks - d.seg_first;
     uint32_t b = blockIdx.x;
-    if (b < resolve_blocks) {
-        uint32_t lo = 0, hi = nreq - 1;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi + 1) >> 1;
-            if (reqs[mid].out_block <= b) lo = mid; else hi = mid - 1;
+    if (b < resolves) {
+        deliver_share(reqs, nreq, d.resolve_blocks, d.segs, d.nseg, d.resolve_first + b);
+    } else if ((b -= resolves) < segs) {
+        deliver_share(reqs, nreq, d.resolve_blocks, d.segs, d.nseg, d.resolve_blocks + d.seg_first + b);
+    } else if ((b -= segs) < d.again_blocks) {
+        const uint32_t n = ldgu(d.redo_ctr, 0);
+        for (uint32_t i = b * DELIVER_THREADS + threadIdx.x; i < n; i += d.again_blocks * DELIVER_THREADS) {
+            const uint32_t slot = ldgu(d.redo_q, i);
+            const uint32_t r = find_req(reqs, nreq, slot >> 6, false);
+            if (r < d.early_reqs) deliver_again(reqs[r], slot);
         }
-        const KReq &r = reqs[lo];
-        const uint32_t at = (b - r.out_block) * RESOLVE_PIXELS + 4u * threadIdx.x;
-        const uint32_t total = r.bgra ? (r.v.width1 - 1u) * (r.v.height1 - 1u) : 0u;
-        if (at < total) resolve_pixels(r, at, min(4u, total - at));
-    } else if ((b -= resolve_blocks) < seg_blocks) {
-        uint32_t lo = 0, hi = nseg - 1;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi + 1) >> 1;
-            if (segs[mid].first_block <= b) lo = mid; else hi = mid - 1;
-        }
-        copy_segment(segs[lo], b - segs[lo].first_block);
     } else {
         for (uint32_t i = threadIdx.x; i < ncounts; i += DELIVER_THREADS) counts_out[i] = counts[i];
     }
@@ -1887,10 +1971,11 @@ static uint64_t sig_hash(const std::vector<uint64_t> &w) {
    request's frame (and hit records) is copied to pixels_host[i] /
    hits_host[i] when given. Returns when the launch is done. Runs without
    the library lock on a server context: only c's own buffers are written,
-   the scenes are read. */
-int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv, uint32_t n, int want_hits,
-                     int persistent, StRayCounts *counts, StFloatPixel *const *pixels_host,
-                     StHitRec *const *hits_host, uint32_t *const *bgra_host, float *kernel_ms) {
+   the scenes are read. The first `plain` requests have no bounce stage and are
+   delivered early (KEarly). */
+static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv, uint32_t n, uint32_t plain,
+                          int want_hits, int persistent, StRayCounts *counts, StFloatPixel *const *pixels_host,
+                          StHitRec *const *hits_host, uint32_t *const *bgra_host, float *kernel_ms) {
     int rc = ensure_init();
     if (rc) return rc;
     if (n == 0) return set_err(ST_ERR_ARG, "no requests");
@@ -2055,6 +2140,10 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
     }
     uint32_t row_base = 0, count_blocks = 0, any_device_ssb = 0, seg = 0;
     KSeg *segs_h = (KSeg *)(st + o_segs);
+    /* the plain requests' tiles and outputs, delivered during the rest's
+       primary stage */
+    KEarly early = {};
+    uint32_t plain_tiles = 0, plain_segs = 0;
     auto deliver = [&](const void *src, void *dst, size_t bytes) {
         segs_h[seg++] = KSeg{(const char *)src, (char *)dst, bytes, seg_blocks, 0};
         seg_blocks += (uint32_t)((bytes + SEG_CHUNK - 1) / SEG_CHUNK);
@@ -2084,8 +2173,8 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
             reqs_h[i].bgra = own_bgra[i] ? bgra_host[i] : (uint32_t *)arena_take(&c->work, (size_t)wpx * 4);
             resolve_blocks += (wpx + RESOLVE_PIXELS - 1) / RESOLVE_PIXELS;
         }
-        if (own_px[i]) deliver(dv.pixels, pixels_host[i], px * 24);
-        if (own_hits[i]) deliver(dv.hits, hits_host[i], px * 16);
+        if (own_px[i]) deliver(dv.pixels, reqs_h[i].px_out = (char *)pixels_host[i], px * 24);
+        if (own_hits[i]) deliver(dv.hits, reqs_h[i].hits_out = (char *)hits_host[i], px * 16);
         if (hv[i].device_ssb) {
             const sm3 &m = hv[i].rotation_matrix_inverted;
             const float rmi[9] = {m.X.x, m.X.y, m.X.z, m.Y.x, m.Y.y, m.Y.z, m.Z.x, m.Z.y, m.Z.z};
@@ -2095,6 +2184,15 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
             any_device_ssb = 1;
         }
         row_base += dv.height1;
+        if (i + 1 == plain) {
+            early.segs = (const KSeg *)(blk + o_segs);
+            early.nreq = plain;
+            early.nseg = seg;
+            early.resolve_blocks = resolve_blocks;
+            early.shares = resolve_blocks + seg_blocks;
+            plain_tiles = dv.tile_base + reqs_h[i].tile_count;
+            plain_segs = seg_blocks;
+        }
     }
     KWave w;
     memset(&w, 0, sizeof w);
@@ -2201,16 +2299,29 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
                            order_blocks);
         HIP_TRY(hipGetLastError());
         HIP_TRY(mark());
-        if (waves4)
-            hipLaunchKernelGGL(k_primary4, dim3(blocks), dim3(BLOCK_THREADS), lds_primary, c->stream,
-                               (const StDScene *)sc_d, (const KReq *)reqs_d, n, tiles, c->tile_counter,
-                               claim_mode, xcd_blocks, ks, km, w, (const uint32_t *)c->tile_order,
-                               c->tile_cost);
-        else
-            hipLaunchKernelGGL(k_primary, dim3(blocks), dim3(BLOCK_THREADS), lds_primary, c->stream,
-                               (const StDScene *)sc_d, (const KReq *)reqs_d, n, tiles, c->tile_counter,
-                               claim_mode, xcd_blocks, ks, km, w, (const uint32_t *)c->tile_order,
-                               c->tile_cost);
+        auto primary = [&](uint32_t first, uint32_t count, uint32_t *counters, const KEarly &e) {
+            const uint32_t nb = std::min(blocks, (count + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK);
+            const uint32_t nblocks = persistent ? nb : blocks;
+            const uint32_t mode = claim_mode == 2u && count >= XCD_MIN_TILES * nblocks * WAVES_PER_BLOCK ? 2u
+                                  : claim_mode ? 1u : 0u;
+            if (waves4)
+                hipLaunchKernelGGL(k_primary4, dim3(nblocks), dim3(BLOCK_THREADS), lds_primary, c->stream,
+                                   (const StDScene *)sc_d, (const KReq *)reqs_d, n, count, counters, mode, xcd_blocks,
+                                   ks, km, w, (const uint32_t *)c->tile_order + first, c->tile_cost, e);
+            else
+                hipLaunchKernelGGL(k_primary, dim3(nblocks), dim3(BLOCK_THREADS), lds_primary, c->stream,
+                                   (const StDScene *)sc_d, (const KReq *)reqs_d, n, count, counters, mode, xcd_blocks,
+                                   ks, km, w, (const uint32_t *)c->tile_order + first, c->tile_cost, e);
+        };
+        static_assert(EARLY_CLAIMS + XCD_CLAIM + 8 * XCD_CLAIM_STRIDE <= CLAIM_WORDS &&
+                          EARLY_CLAIMS >= XCD_CLAIM + 8 * XCD_CLAIM_STRIDE,
+                      "the second primary kernel's claim counters are words of their own");
+        if (plain_tiles) {
+            primary(0, plain_tiles, c->tile_counter, KEarly{});
+            primary(plain_tiles, tiles - plain_tiles, c->tile_counter + EARLY_CLAIMS, early);
+        } else {
+            primary(0, tiles, c->tile_counter, KEarly{});
+        }
         HIP_TRY(hipGetLastError());
         HIP_TRY(mark());
         /* the rest of the depth loop: the bounce stage reads its queue
@@ -2297,8 +2408,19 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
     }
     /* this launch's tile times are now what tile_cost will hold */
     c->tile_sig = tile_sig;
-    hipLaunchKernelGGL(k_deliver, dim3(resolve_blocks + seg_blocks + 1), dim3(DELIVER_THREADS), 0, c->stream,
-                       (const KReq *)reqs_d, n, resolve_blocks, (const KSeg *)(blk + o_segs), nseg, seg_blocks,
+    KDeliver d;
+    d.segs = (const KSeg *)(blk + o_segs);
+    d.nseg = nseg;
+    d.resolve_first = early.resolve_blocks;
+    d.resolve_blocks = resolve_blocks;
+    d.seg_first = plain_segs;
+    d.seg_blocks = seg_blocks;
+    d.early_reqs = early.nreq;
+    d.again_blocks = early.nreq ? 8u : 0u;
+    d.redo_ctr = w.redo_ctr;
+    d.redo_q = w.redo_q;
+    hipLaunchKernelGGL(k_deliver, dim3(resolve_blocks - d.resolve_first + seg_blocks - d.seg_first + d.again_blocks + 1),
+                       dim3(DELIVER_THREADS), 0, c->stream, (const KReq *)reqs_d, n, d,
                        (const unsigned long long *)cnt_d, (unsigned long long *)(c->staging_dev + o_readback),
                        3 * n + 2);
     HIP_TRY(hipGetLastError());
@@ -2329,6 +2451,73 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
     c->stage_n = marks ? marks - 1 : 0;
     for (uint32_t k = 0; k < c->stage_n; k++)
         HIP_TRY(hipEventElapsedTime(&c->stage_ms[k], c->stage_ev[k], c->stage_ev[k + 1]));
+    return rc;
+}
+
+/* A launch of plain requests (no bounce stage) with enough to deliver and of
+   others with enough to render meanwhile (EARLY_MIN_BYTES) runs in an order
+   of its own, the plain ones first (KEarly); any other in the caller's. A
+   captured graph keeps its outputs out of the graph, so its launches are not
+   split; neither are those with an order of tiles of their own
+   (StTuning.cost_order 1) or one wave per tile. */
+int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv, uint32_t n, int want_hits,
+                     int persistent, StRayCounts *counts, StFloatPixel *const *pixels_host,
+                     StHitRec *const *hits_host, uint32_t *const *bgra_host, float *kernel_ms) {
+    auto straight = [&]() {
+        return launch_ordered(c, scenes, hv, n, 0, want_hits, persistent, counts, pixels_host, hits_host, bgra_host,
+                              kernel_ms);
+    };
+    int rc = ensure_init();
+    if (rc) return rc;
+    uint32_t cost_order;
+    {
+        RT_LOCK;
+        cost_order = g.tune.cost_order;
+    }
+    if (n < 2 || !persistent || c->graph_mode || cost_order == 1u) return straight();
+    auto shaded = [&](uint32_t i) { return hv[i].dv.mode == ST_MODE_BEAUTY && hv[i].dv.depth > 1; };
+    uint64_t out = 0, px_shaded = 0;
+    for (uint32_t i = 0; i < n; i++) {
+        const uint64_t w1 = hv[i].dv.width1, h1 = hv[i].dv.height1, px = w1 * h1;
+        if (!scenes[i] || !scenes[i]->host || !scenes[i]->dbuf || w1 < 2 || h1 < 2) return straight();
+        if (shaded(i)) {
+            px_shaded += px;
+            continue;
+        }
+        if (bgra_host && bgra_host[i] && deliverable(bgra_host[i], (w1 - 1) * (h1 - 1) * 4))
+            out += (w1 - 1) * (h1 - 1) * 4;
+        if (pixels_host && pixels_host[i] && deliverable(pixels_host[i], px * 24)) out += px * 24;
+        if (want_hits && hits_host && hits_host[i] && deliverable(hits_host[i], px * 16)) out += px * 16;
+    }
+    if (out < EARLY_MIN_BYTES || px_shaded < EARLY_MIN_PIXELS) return straight();
+    std::vector<uint32_t> at(n);   /* launch order -> the caller's */
+    uint32_t plain = 0, k = 0;
+    for (uint32_t i = 0; i < n; i++)
+        if (!shaded(i)) at[plain++] = i;
+    k = plain;
+    for (uint32_t i = 0; i < n; i++)
+        if (shaded(i)) at[k++] = i;
+    std::vector<StSceneHandle *> o_scenes(n);
+    std::vector<StHostView> o_hv(n);
+    std::vector<StRayCounts> o_counts(counts ? n : 0);
+    std::vector<StFloatPixel *> o_px(pixels_host ? n : 0);
+    std::vector<StHitRec *> o_hits(hits_host ? n : 0);
+    std::vector<uint32_t *> o_bgra(bgra_host ? n : 0);
+    for (uint32_t i = 0; i < n; i++) {
+        o_scenes[i] = scenes[at[i]];
+        o_hv[i] = hv[at[i]];
+        if (counts) o_counts[i] = counts[at[i]];
+        if (pixels_host) o_px[i] = pixels_host[at[i]];
+        if (hits_host) o_hits[i] = hits_host[at[i]];
+        if (bgra_host) o_bgra[i] = bgra_host[at[i]];
+    }
+    rc = launch_ordered(c, o_scenes.data(), o_hv.data(), n, plain, want_hits, persistent,
+                        counts ? o_counts.data() : NULL, pixels_host ? o_px.data() : NULL,
+                        hits_host ? o_hits.data() : NULL, bgra_host ? o_bgra.data() : NULL, kernel_ms);
+    for (uint32_t i = 0; i < n; i++) {
+        hv[at[i]].dv = o_hv[i].dv;
+        if (counts) counts[at[i]] = o_counts[i];
+    }
     return rc;
 }
 
@@ -2531,7 +2720,7 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
     HIP_TRY(hipGetLastError());
     hipLaunchKernelGGL(k_primary, dim3(blocks), dim3(BLOCK_THREADS), lds_primary, stream, sc_d, reqs_d, 1u, tiles, ctr,
                        claim_mode, xcd_blocks, ks, km, w,
-                       (const uint32_t *)(base + o_order), (uint32_t *)(base + o_cost));
+                       (const uint32_t *)(base + o_order), (uint32_t *)(base + o_cost), KEarly{});
     HIP_TRY(hipGetLastError());
     if (beauty && dv.depth > 1) {
         const uint32_t b_bounce = resident_blocks(reinterpret_cast<const void *>(k_bounce), lds);
@@ -2544,8 +2733,12 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
         hipLaunchKernelGGL(k_counts, dim3((tiles + COUNT_TILES - 1) / COUNT_TILES), dim3(256), 0, stream, reqs_d, 1u,
                            (const uint32_t *)w.counts);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(k_deliver, dim3(seg_blocks + 1), dim3(DELIVER_THREADS), 0, stream, reqs_d, 1u, 0u,
-                       (const KSeg *)(base + o_segs), nseg, seg_blocks, (const unsigned long long *)cnt_d,
+    KDeliver d = {};
+    d.segs = (const KSeg *)(base + o_segs);
+    d.nseg = nseg;
+    d.seg_blocks = seg_blocks;
+    hipLaunchKernelGGL(k_deliver, dim3(seg_blocks + 1), dim3(DELIVER_THREADS), 0, stream, reqs_d, 1u, d,
+                       (const unsigned long long *)cnt_d,
                        (unsigned long long *)(g_noalloc_host_dev + ST_NOALLOC_COUNTS), 5u);
     HIP_TRY(hipGetLastError());
     if (!own_px) HIP_TRY(hipMemcpyAsync(pixels, base + o_pix, px * 24, hipMemcpyDeviceToHost, stream));
@@ -2780,9 +2973,10 @@ extern "C" int st_resolve_bgra8(const StFloatPixel *grid, uint32_t grid_w, uint3
     HIP_TRY(hipMemcpyAsync(grid_d, grid, gbytes, hipMemcpyHostToDevice, g.main.stream));
     HIP_TRY(hipMemcpyAsync(req_d, req_h, sizeof(KReq), hipMemcpyHostToDevice, g.main.stream));
     const uint32_t blocks = (uint32_t)((opx + RESOLVE_PIXELS - 1) / RESOLVE_PIXELS);
-    hipLaunchKernelGGL(k_deliver, dim3(blocks), dim3(DELIVER_THREADS), 0, g.main.stream, (const KReq *)req_d, 1u,
-                       blocks, (const KSeg *)NULL, 0u, 0u, (const unsigned long long *)NULL,
-                       (unsigned long long *)NULL, 0u);
+    KDeliver d = {};
+    d.resolve_blocks = blocks;
+    hipLaunchKernelGGL(k_deliver, dim3(blocks), dim3(DELIVER_THREADS), 0, g.main.stream, (const KReq *)req_d, 1u, d,
+                       (const unsigned long long *)NULL, (unsigned long long *)NULL, 0u);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(out, out_d, opx * 4, hipMemcpyDeviceToHost, g.main.stream));
     HIP_TRY(hipStreamSynchronize(g.main.stream));

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import slimtracin_amd as st
-from slimtracin_amd.scene import HIT_DTYPE, MODE_BEAUTY, MODE_NORMALS, PIXEL_DTYPE, make_view
+from slimtracin_amd.scene import HIT_DTYPE, MODE_BEAUTY, MODE_DEPTH, MODE_NORMALS, MODE_UVS, PIXEL_DTYPE, make_view
 
 pytestmark = pytest.mark.gpu
 
@@ -90,3 +90,60 @@ def test_grids_and_hits(scene, offset, call):
         assert pix[i].tobytes() == want_p[i].tobytes() and hits[i].tobytes() == want_h[i].tobytes()
         assert (counts[i].shadow, counts[i].bounce) == (want_c[i].shadow, want_c[i].bounce)
     assert _guards_stand(pb, ps) and _guards_stand(hb, hs)
+
+
+@pytest.mark.parametrize("abandon", [0, 48])
+@pytest.mark.parametrize("call", ["windows", "grids"])
+def test_plain_requests_of_a_mixed_launch(call, abandon):
+    """Requests without a bounce stage are delivered while the Beauty ones render; the ones that the redo stage then
+    changes (abandon: a small step limit makes some) are delivered again. Each request alone has none to overlap with."""
+    ds = st.DeviceScene(st.gen_pbr(3, 20), mesh_lbvh=True)
+    sizes = [(1201, 701), (1, 1), (1600, 900), (640, 363), (1601, 900), (17, 5), (1024, 640)]
+    modes = [MODE_BEAUTY, MODE_NORMALS, MODE_NORMALS, MODE_DEPTH, MODE_BEAUTY, MODE_BEAUTY, MODE_UVS]
+    if call == "windows":   # 4 bytes a pixel, where a grid and its hit records have 40: as many bytes as those
+        sizes += [(3201, 2003), (3199, 1999)]
+        modes += [MODE_UVS, MODE_NORMALS]
+    grid = [(w + 1) * (h + 1) for w, h in sizes]
+    views = np.concatenate([make_view(width=w, height=h, mode=m, depth=0 if w == 17 else 2,
+                                     position=(0.0, 3.0, -9.0), pitch=-0.1) for (w, h), m in zip(sizes, modes)])
+    n = len(views)
+    try:
+        st.debug_redo(abandon, 1 if abandon else 0)
+        redone = 0
+        if call == "windows":
+            want, want_c = [], []
+            for i in range(n):
+                a, c = st.render_batch_bgra8([ds], views[i:i + 1])
+                redone += st.last_redo_count()
+                want.append(a[0])
+                want_c += c
+            block, spans = _guarded([w * h for w, h in sizes], 4, 4)
+            outs = [block[a:b].view(np.uint32) for a, b in spans]
+            got, counts = st.render_batch_bgra8([ds] * n, views, outs=outs)
+            assert all((g == w).all() for g, w in zip(got, want))
+            assert _guards_stand(block, spans)
+        else:
+            want_p, want_h, want_c = [], [], []
+            for i in range(n):
+                p, h, c = st.render_batch([ds], views[i:i + 1], hits=True)
+                redone += st.last_redo_count()
+                want_p += p
+                want_h += h
+                want_c += c
+            pb, ps = _guarded(grid, PIXEL_DTYPE.itemsize, 8)
+            hb, hs = _guarded(grid, HIT_DTYPE.itemsize, 8)
+            pix = [pb[a:b].view(PIXEL_DTYPE) for a, b in ps]
+            hits = [hb[a:b].view(HIT_DTYPE) for a, b in hs]
+            counts = (st.RayCounts * n)()
+            rc = st.lib().st_render_batch((C.c_void_p * n)(*[ds.handle] * n), views.ctypes.data_as(C.c_void_p),
+                                          C.c_uint32(n), (C.c_void_p * n)(*[p.ctypes.data for p in pix]),
+                                          (C.c_void_p * n)(*[h.ctypes.data for h in hits]), counts, C.c_uint32(1))
+            assert rc == 0
+            for i in range(n):
+                assert pix[i].tobytes() == want_p[i].tobytes() and hits[i].tobytes() == want_h[i].tobytes()
+            assert _guards_stand(pb, ps) and _guards_stand(hb, hs)
+        assert [(c.primary, c.shadow, c.bounce) for c in counts] == [(c.primary, c.shadow, c.bounce) for c in want_c]
+        assert not abandon or redone
+    finally:
+        st.debug_redo(0, 0)
+        ds.close()
