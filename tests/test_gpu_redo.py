@@ -122,6 +122,31 @@ def test_degenerate_rays_take_the_redo_stage():
         assert _check(blob, view, f"degenerate/m{mode}", lbvh=True, want_blob=want) > 0
 
 
+@pytest.mark.parametrize("triangles", [2000, 20000, 200000])
+@pytest.mark.parametrize("size", [(1, 1), (65, 49)])
+def test_short_and_long_jobs_equal_a_lone_traversal(triangles, size):
+    """Jobs that the leader ends alone (ordinary rays) and jobs that it opens to the group's helpers (degenerate
+    ones), in one pixel's path: the frame, hits and counts of the main stages that never give up."""
+    blob = st.gen_mesh_scene(5, triangles)
+    prims = blob_prims(blob)
+    prims[0]["rotation"] = (0.0, 0.0, 0.0, 1.0)
+    prims[0]["flags"] &= ~np.uint32(IS_ROTATED)
+    ds = st.DeviceScene(blob_with_prims(blob, prims), mesh_binned=True)
+    view = make_view(width=size[0], height=size[1], mode=MODE_BEAUTY, depth=3, position=(0.0, 3.0, -10.0))
+    try:
+        st.debug_redo(1 << 30, 1 << 30)
+        want = st.render(ds, view)
+        assert st.last_redo_count() == 0
+        st.debug_redo(2, 16)
+        got = st.render(ds, view)
+        assert st.last_redo_count() > 0
+    finally:
+        st.debug_redo(0, 0)
+        ds.close()
+    assert got[0].tobytes() == want[0].tobytes() and got[1].tobytes() == want[1].tobytes()
+    assert (got[2].shadow, got[2].bounce) == (want[2].shadow, want[2].bounce)
+
+
 def test_batched_redo_equals_plain(redo_everything):
     """A batch whose pixels go through the redo stage equals the plain
     launches of its requests."""
