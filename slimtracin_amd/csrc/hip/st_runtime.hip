@@ -39,8 +39,8 @@
  *                   each pixel's whole path again by a group of blocks,
  *                   with large mesh traversals split across the group.
  *   k_counts        per-request shadow/bounce ray totals.
- *   k_deliver       window images resolved, grids, hit records and counts
- *                   written to where the caller wants them.
+ *   k_deliver       window images resolved straight to where the caller
+ *                   wants them, and the counts.
  */
 #include <hip/hip_runtime.h>
 
@@ -116,9 +116,6 @@ struct KReq {
     uint32_t out_block;    /* first block of the display resolve for this request (k_deliver) */
     uint32_t count_block;  /* first block of k_counts for this request */
     uint32_t *bgra;        /* window image (width1-1)*(height1-1), or NULL */
-    /* where the device itself writes the traced grid and the hit records
-       (page-locked host memory), or NULL */
-    char *px_out, *hits_out;
     uint64_t pad2;
     /* device SSB pass (k_ssb) when device_ssb: camera rotation_matrix_inverted
        (rows X, Y, Z) and focal length; ssb_raw / ssb_flags optionally receive
@@ -496,63 +493,24 @@ __device__ static inline void resolve_pixels(const KReq &r, uint32_t at, uint32_
     }
 }
 
-/* What a launch hands over, in one launch at its end: window images (the
-   display resolve, straight to where they go), traced grids and hit records
-   (16 KB of a segment per block), and the ray counts. Destinations are
-   page-locked host memory that the device writes over the link, or device
-   buffers that are copied on from there. Bound by the link (50 of its 57 GB/s):
-   160 window images, 189 MB, take 3.8 ms; resolved into device memory
-   (0.7 ms) and copied by a call each they took 7. Plain requests of a mixed
-   launch go out earlier (KEarly). */
+/* Window images, resolved straight to where they go: page-locked host memory
+   that the device writes over the link, or a device buffer that is copied on
+   from there. Bound by the link (50 of its 57 GB/s): 160 window images, 189
+   MB, take 3.8 ms; resolved into device memory (0.7 ms) and copied by a call
+   each they took 7. Plain requests of a mixed launch go out earlier (KEarly).
+   Block `b` of the launch's resolve. */
 #define DELIVER_THREADS 256u
 #define RESOLVE_PIXELS (4u * DELIVER_THREADS)   /* per block */
-#define SEG_CHUNK 16384u
-struct KSeg {
-    const char *src;
-    char *dst;
-    uint64_t bytes;        /* a multiple of 4, as are both addresses */
-    uint32_t first_block;
-    uint32_t pad;
-};
-__device__ static inline void copy_segment(const KSeg &g, uint32_t chunk) {
-    const uint64_t at = (uint64_t)chunk * SEG_CHUNK;
-    const uint32_t n = (uint32_t)min((uint64_t)SEG_CHUNK, g.bytes - at);
-    const char *src = g.src + at;
-    char *dst = g.dst + at;
-    if ((((uintptr_t)src | (uintptr_t)dst) & 15u) == 0) {
-        for (uint32_t i = threadIdx.x * 16u; i + 16u <= n; i += DELIVER_THREADS * 16u)
-            *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(src + i);
-        const uint32_t tail = n & ~15u;
-        for (uint32_t i = tail + threadIdx.x * 4u; i < n; i += DELIVER_THREADS * 4u)
-            *reinterpret_cast<uint32_t *>(dst + i) = *reinterpret_cast<const uint32_t *>(src + i);
-    } else {
-        for (uint32_t i = threadIdx.x * 4u; i < n; i += DELIVER_THREADS * 4u)
-            *reinterpret_cast<uint32_t *>(dst + i) = *reinterpret_cast<const uint32_t *>(src + i);
+__device__ static inline void resolve_share(const KReq *reqs, uint32_t nreq, uint32_t b) {
+    uint32_t lo = 0, hi = nreq - 1;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi + 1) >> 1;
+        if (reqs[mid].out_block <= b) lo = mid; else hi = mid - 1;
     }
-}
-/* Share `b` of a launch's delivery: resolve shares first, then segments'. */
-__device__ static inline void deliver_share(const KReq *reqs, uint32_t nreq, uint32_t resolve_blocks,
-                                            const KSeg *segs, uint32_t nseg, uint32_t b) {
-    uint32_t lo = 0;
-    if (b < resolve_blocks) {
-        uint32_t hi = nreq - 1;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi + 1) >> 1;
-            if (reqs[mid].out_block <= b) lo = mid; else hi = mid - 1;
-        }
-        const KReq &r = reqs[lo];
-        const uint32_t at = (b - r.out_block) * RESOLVE_PIXELS + 4u * threadIdx.x;
-        const uint32_t total = r.bgra ? (r.v.width1 - 1u) * (r.v.height1 - 1u) : 0u;
-        if (at < total) resolve_pixels(r, at, min(4u, total - at));
-    } else {
-        b -= resolve_blocks;
-        uint32_t hi = nseg - 1;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi + 1) >> 1;
-            if (segs[mid].first_block <= b) lo = mid; else hi = mid - 1;
-        }
-        copy_segment(segs[lo], b - segs[lo].first_block);
-    }
+    const KReq &r = reqs[lo];
+    const uint32_t at = (b - r.out_block) * RESOLVE_PIXELS + 4u * threadIdx.x;
+    const uint32_t total = r.bgra ? (r.v.width1 - 1u) * (r.v.height1 - 1u) : 0u;
+    if (at < total) resolve_pixels(r, at, min(4u, total - at));
 }
 
 /* Delivery during the primary stage. A launch whose requests include both
@@ -576,9 +534,8 @@ __device__ static inline void deliver_share(const KReq *reqs, uint32_t nreq, uin
 #define EARLY_MIN_BYTES (48ull << 20)
 #define EARLY_MIN_PIXELS (1u << 21)
 struct KEarly {
-    const KSeg *segs;
-    uint32_t nreq, nseg;               /* the plain requests and their segments: the first of the launch's */
-    uint32_t resolve_blocks, shares;   /* shares 0: nothing to deliver */
+    uint32_t nreq;      /* the plain requests: the first of the launch's */
+    uint32_t shares;    /* their resolve blocks; 0: nothing to deliver */
 };
 
 /* Traversal stacks live in LDS, one column per lane (no bank conflicts):
@@ -626,7 +583,7 @@ primary_stage(const StDScene *__restrict__ scenes, const KReq *__restrict__ reqs
               uint32_t *__restrict__ tile_cost, const KEarly &early) {
     if (blockIdx.x < EARLY_BLOCKS)
         for (uint32_t s = blockIdx.x; s < early.shares; s += min(gridDim.x, EARLY_BLOCKS))
-            deliver_share(reqs, early.nreq, early.resolve_blocks, early.segs, early.nseg, s);
+            resolve_share(reqs, early.nreq, s);
     ST_LDS_STACKS(scene_entries, mesh_entries);
     const DStacks stk = {scene_stack, mesh_stack, nullptr};
     /* One call site, so primary_tile is inlined once. Persistent (1): waves
@@ -1177,53 +1134,39 @@ __global__ void __launch_bounds__(64) k_pick(const StDScene *__restrict__ scenes
     stg2(o, 2, __float_as_uint(out[4]), __float_as_uint(out[5]));
 }
 
-/* One redone pixel of a request whose outputs went out before the redo
-   stage: its grid and hit records and the window pixels it is a corner of. */
-__device__ static inline void deliver_again(const KReq &r, uint32_t slot) {
+/* The window pixels that a redone pixel is a corner of, of a request whose
+   image went out before the redo stage. */
+__device__ static inline void resolve_again(const KReq &r, uint32_t slot) {
     uint32_t x, y;
-    if (!tile_pixel(r.v, slot >> 6, slot & 63u, x, y)) return;
-    const size_t pix = (size_t)y * r.v.width1 + x;
-    if (r.px_out)
-        for (uint32_t k = 0; k < 6; k++)
-            reinterpret_cast<uint32_t *>(r.px_out)[pix * 6 + k] = reinterpret_cast<const uint32_t *>(r.v.pixels)[pix * 6 + k];
-    if (r.hits_out)
-        for (uint32_t k = 0; k < 4; k++)
-            reinterpret_cast<uint32_t *>(r.hits_out)[pix * 4 + k] = reinterpret_cast<const uint32_t *>(r.v.hits)[pix * 4 + k];
-    if (r.bgra) {
-        const uint32_t w = r.v.width1 - 1u, h = r.v.height1 - 1u;
-        for (uint32_t j = 0; j < 4; j++) {
-            const uint32_t wx = x - (j & 1u), wy = y - (j >> 1);
-            if (wx < w && wy < h) resolve_pixels(r, wy * w + wx, 1u);
-        }
+    if (!r.bgra || !tile_pixel(r.v, slot >> 6, slot & 63u, x, y)) return;
+    const uint32_t w = r.v.width1 - 1u, h = r.v.height1 - 1u;
+    for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t wx = x - (j & 1u), wy = y - (j >> 1);
+        if (wx < w && wy < h) resolve_pixels(r, wy * w + wx, 1u);
     }
 }
 
-/* `shares` shares from first.resolve on (window images) and from first.seg on
-   (segments), the counts, and the redone pixels of the requests that went out
-   before (early_reqs, the launch's first). */
+/* What a launch hands over at its end: the window images from block
+   resolve_first on, the redone pixels of the images before (the first
+   early_reqs requests'), and the counts. */
 struct KDeliver {
-    const KSeg *segs;
-    uint32_t nseg;
-    uint32_t resolve_first, resolve_blocks;   /* shares already out, and of all requests */
-    uint32_t seg_first, seg_blocks;
+    uint32_t resolve_first, resolve_blocks;
     uint32_t early_reqs, again_blocks;
     const uint32_t *redo_ctr, *redo_q;
 };
 __global__ void __launch_bounds__(DELIVER_THREADS) k_deliver(const KReq *__restrict__ reqs, uint32_t nreq, KDeliver d,
                                                              const unsigned long long *counts,
                                                              unsigned long long *counts_out, uint32_t ncounts) {
-    const uint32_t resolves = d.resolve_blocks - d.resolve_first, segs = d.seg_blocks - d.seg_first;
+    const uint32_t resolves = d.resolve_blocks - d.resolve_first;
     uint32_t b = blockIdx.x;
     if (b < resolves) {
-        deliver_share(reqs, nreq, d.resolve_blocks, d.segs, d.nseg, d.resolve_first + b);
-    } else if ((b -= resolves) < segs) {
-        deliver_share(reqs, nreq, d.resolve_blocks, d.segs, d.nseg, d.resolve_blocks + d.seg_first + b);
-    } else if ((b -= segs) < d.again_blocks) {
+        resolve_share(reqs, nreq, d.resolve_first + b);
+    } else if ((b -= resolves) < d.again_blocks) {
         const uint32_t n = ldgu(d.redo_ctr, 0);
         for (uint32_t i = b * DELIVER_THREADS + threadIdx.x; i < n; i += d.again_blocks * DELIVER_THREADS) {
             const uint32_t slot = ldgu(d.redo_q, i);
             const uint32_t r = find_req(reqs, nreq, slot >> 6, false);
-            if (r < d.early_reqs) deliver_again(reqs[r], slot);
+            if (r < d.early_reqs) resolve_again(reqs[r], slot);
         }
     } else {
         for (uint32_t i = threadIdx.x; i < ncounts; i += DELIVER_THREADS) counts_out[i] = counts[i];
@@ -1263,7 +1206,7 @@ __global__ void k_zero_u64(unsigned long long *p, uint32_t n) {
 /* ---- page-locked host memory ---------------------------------------------- */
 
 /* The library's live page-locked blocks (st_host_alloc), by address: outputs
-   inside one are written by the device itself (k_deliver). */
+   inside one are written by the device itself (deliverable). */
 static std::mutex g_pin_mu;
 static std::map<uintptr_t, size_t> &g_pinned = *new std::map<uintptr_t, size_t>;   /* lives as long as the process */
 
@@ -1274,10 +1217,19 @@ static bool pinned_range(const void *p, size_t bytes) {
     --it;
     return (uintptr_t)p + bytes <= it->first + it->second;
 }
-/* an output that k_deliver can write: page-locked, and of 4-byte words */
-static bool deliverable(const void *p, size_t bytes) {
-    return ((uintptr_t)p & 3u) == 0 && (bytes & 3u) == 0 && pinned_range(p, bytes);
+/* Outputs that the device writes itself: page-locked, and aligned for the
+   kernels' stores. Window images by k_deliver; grids and hit records by the
+   kernels that make them, so that they go over the link while other pixels
+   render (every pixel is written once, again only by the redo stage).
+   Written by a copy in k_deliver instead, frames took 1185 us against 985
+   (799x601 pixels of a 20k-triangle scene, Beauty), 319 against 277 (640x480
+   of implicit primitives) and 1615 against 1450 (1283x719 normals). */
+static bool deliverable(const void *p, size_t bytes, size_t align) {
+    return ((uintptr_t)p & (align - 1)) == 0 && pinned_range(p, bytes);
 }
+#define IMAGE_ALIGN 4u
+#define GRID_ALIGN 8u    /* finish_pixel */
+#define HITS_ALIGN 16u   /* primary_pixel */
 
 /* ---- context ------------------------------------------------------------ */
 
@@ -2002,7 +1954,7 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
     /* outputs that the device writes itself (page-locked); the others are
        copied on after the launch */
     std::vector<char> own_px(n), own_hits(n), own_bgra(n);
-    uint32_t nseg = 0, seg_blocks = 0, resolve_blocks = 0;
+    uint32_t resolve_blocks = 0;
     for (uint32_t i = 0; i < n; i++) {
         StSceneHandle *s = scenes[i];
         if (!s || !s->host || !s->dbuf) return set_err(ST_ERR_ARG, "request %u has no resident scene", i);
@@ -2011,17 +1963,19 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
         if (k == nuniq) uniq[nuniq++] = s;
         scene_idx[i] = k;
         size_t px = (size_t)hv[i].dv.width1 * hv[i].dv.height1;
-        per_req_out += round256((size_t)hv[i].dv.height1 * ST_DIR_MARKS(hv[i].dv.width1) * 16) + round256(px * 24) +
-                       (want_hits ? round256(px * 16) : 0);
+        per_req_out += round256((size_t)hv[i].dv.height1 * ST_DIR_MARKS(hv[i].dv.width1) * 16);
         if (bgra_host && bgra_host[i]) {
             if (hv[i].dv.width1 < 2 || hv[i].dv.height1 < 2) return set_err(ST_ERR_ARG, "request %u: empty window", i);
             const size_t wb = (size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4;
-            own_bgra[i] = deliverable(bgra_host[i], wb);
+            own_bgra[i] = deliverable(bgra_host[i], wb, IMAGE_ALIGN);
             if (!own_bgra[i]) per_req_out += round256(wb);
         }
-        own_px[i] = pixels_host && pixels_host[i] && deliverable(pixels_host[i], px * 24);
-        own_hits[i] = want_hits && hits_host && hits_host[i] && deliverable(hits_host[i], px * 16);
-        nseg += (uint32_t)own_px[i] + (uint32_t)own_hits[i];
+        /* (the resolve reads the grid: it stays in device memory) */
+        own_px[i] = pixels_host && pixels_host[i] && !(bgra_host && bgra_host[i]) &&
+                    deliverable(pixels_host[i], px * 24, GRID_ALIGN);
+        own_hits[i] = want_hits && hits_host && hits_host[i] && deliverable(hits_host[i], px * 16, HITS_ALIGN);
+        if (!own_px[i]) per_req_out += round256(px * 24);
+        if (want_hits && !own_hits[i]) per_req_out += round256(px * 16);
         const uint32_t tw = 1u << tune.tile_shift, th = 64u >> tune.tile_shift;
         hv[i].dv.tile_shift = tune.tile_shift;
         hv[i].dv.tiles_x = (hv[i].dv.width1 + tw - 1) / tw;
@@ -2044,8 +1998,6 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
         rect_off[i] = up;
         up += round256((scenes[i]->host->prim_count + 1) * 16ull);
     }
-    const size_t o_segs = up;
-    up += round256(nseg * sizeof(KSeg));
     /* wavefront buffers of the Beauty depth loop: levels = largest depth,
        shadow planes = largest light count among Beauty requests */
     uint32_t levels = 0, lmax = 1;
@@ -2138,16 +2090,11 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
         sc_h[k].spill_s = spill_s;
         sc_h[k].spill_m = spill_m;
     }
-    uint32_t row_base = 0, count_blocks = 0, any_device_ssb = 0, seg = 0;
-    KSeg *segs_h = (KSeg *)(st + o_segs);
-    /* the plain requests' tiles and outputs, delivered during the rest's
+    uint32_t row_base = 0, count_blocks = 0, any_device_ssb = 0;
+    /* the plain requests' tiles and images, delivered during the rest's
        primary stage */
     KEarly early = {};
-    uint32_t plain_tiles = 0, plain_segs = 0;
-    auto deliver = [&](const void *src, void *dst, size_t bytes) {
-        segs_h[seg++] = KSeg{(const char *)src, (char *)dst, bytes, seg_blocks, 0};
-        seg_blocks += (uint32_t)((bytes + SEG_CHUNK - 1) / SEG_CHUNK);
-    };
+    uint32_t plain_tiles = 0;
     for (uint32_t i = 0; i < n; i++) {
         size_t px = (size_t)hv[i].dv.width1 * hv[i].dv.height1;
         StDView &dv = hv[i].dv;
@@ -2158,8 +2105,8 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
         dv.row_starts = (const float *)(blk + rs_off[i]);
         dv.rects = (const int32_t *)(blk + rect_off[i]);
         dv.dir_marks = (float *)arena_take(&c->work, (size_t)dv.height1 * ST_DIR_MARKS(dv.width1) * 16);
-        dv.pixels = arena_take(&c->work, px * 24);
-        dv.hits = want_hits ? arena_take(&c->work, px * 16) : NULL;
+        dv.pixels = own_px[i] ? (void *)pixels_host[i] : arena_take(&c->work, px * 24);
+        dv.hits = own_hits[i] ? (void *)hits_host[i] : want_hits ? arena_take(&c->work, px * 16) : NULL;
         dv.counters = cnt_d + 3 * i;
         memset(&reqs_h[i], 0, sizeof(KReq));
         reqs_h[i].v = dv;
@@ -2173,8 +2120,6 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
             reqs_h[i].bgra = own_bgra[i] ? bgra_host[i] : (uint32_t *)arena_take(&c->work, (size_t)wpx * 4);
             resolve_blocks += (wpx + RESOLVE_PIXELS - 1) / RESOLVE_PIXELS;
         }
-        if (own_px[i]) deliver(dv.pixels, reqs_h[i].px_out = (char *)pixels_host[i], px * 24);
-        if (own_hits[i]) deliver(dv.hits, reqs_h[i].hits_out = (char *)hits_host[i], px * 16);
         if (hv[i].device_ssb) {
             const sm3 &m = hv[i].rotation_matrix_inverted;
             const float rmi[9] = {m.X.x, m.X.y, m.X.z, m.Y.x, m.Y.y, m.Y.z, m.Z.x, m.Z.y, m.Z.z};
@@ -2185,13 +2130,9 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
         }
         row_base += dv.height1;
         if (i + 1 == plain) {
-            early.segs = (const KSeg *)(blk + o_segs);
             early.nreq = plain;
-            early.nseg = seg;
-            early.resolve_blocks = resolve_blocks;
-            early.shares = resolve_blocks + seg_blocks;
+            early.shares = resolve_blocks;
             plain_tiles = dv.tile_base + reqs_h[i].tile_count;
-            plain_segs = seg_blocks;
         }
     }
     KWave w;
@@ -2375,9 +2316,12 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
                                      (uint64_t)(uintptr_t)w.sorted_q, (uint64_t)(uintptr_t)spill, spill_s, spill_m};
         for (uint32_t i = 0; i < n; i++) {
             const StDView &dv = reqs_h[i].v;
+            /* outputs in the caller's memory come with the upload, as the
+               views do: other addresses replay the same graph */
             sig.insert(sig.end(), {dv.width1, dv.height1, dv.mode, dv.depth, dv.tile_shift,
-                                   (uint64_t)(uintptr_t)dv.dir_marks, (uint64_t)(uintptr_t)dv.pixels,
-                                   (uint64_t)(uintptr_t)dv.hits, (uint64_t)(uintptr_t)reqs_h[i].bgra});
+                                   (uint64_t)(uintptr_t)dv.dir_marks, own_px[i] ? 0 : (uint64_t)(uintptr_t)dv.pixels,
+                                   own_hits[i] ? 0 : (uint64_t)(uintptr_t)dv.hits,
+                                   (uint64_t)(uintptr_t)reqs_h[i].bgra});
         }
         if (!c->graph_exec || sig != c->graph_sig) {
             if (c->graph_exec) {
@@ -2409,17 +2353,13 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
     /* this launch's tile times are now what tile_cost will hold */
     c->tile_sig = tile_sig;
     KDeliver d;
-    d.segs = (const KSeg *)(blk + o_segs);
-    d.nseg = nseg;
-    d.resolve_first = early.resolve_blocks;
+    d.resolve_first = early.shares;
     d.resolve_blocks = resolve_blocks;
-    d.seg_first = plain_segs;
-    d.seg_blocks = seg_blocks;
     d.early_reqs = early.nreq;
     d.again_blocks = early.nreq ? 8u : 0u;
     d.redo_ctr = w.redo_ctr;
     d.redo_q = w.redo_q;
-    hipLaunchKernelGGL(k_deliver, dim3(resolve_blocks - d.resolve_first + seg_blocks - d.seg_first + d.again_blocks + 1),
+    hipLaunchKernelGGL(k_deliver, dim3(resolve_blocks - d.resolve_first + d.again_blocks + 1),
                        dim3(DELIVER_THREADS), 0, c->stream, (const KReq *)reqs_d, n, d,
                        (const unsigned long long *)cnt_d, (unsigned long long *)(c->staging_dev + o_readback),
                        3 * n + 2);
@@ -2484,10 +2424,8 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
             px_shaded += px;
             continue;
         }
-        if (bgra_host && bgra_host[i] && deliverable(bgra_host[i], (w1 - 1) * (h1 - 1) * 4))
+        if (bgra_host && bgra_host[i] && deliverable(bgra_host[i], (w1 - 1) * (h1 - 1) * 4, IMAGE_ALIGN))
             out += (w1 - 1) * (h1 - 1) * 4;
-        if (pixels_host && pixels_host[i] && deliverable(pixels_host[i], px * 24)) out += px * 24;
-        if (want_hits && hits_host && hits_host[i] && deliverable(hits_host[i], px * 16)) out += px * 16;
     }
     if (out < EARLY_MIN_BYTES || px_shaded < EARLY_MIN_PIXELS) return straight();
     std::vector<uint32_t> at(n);   /* launch order -> the caller's */
@@ -2589,8 +2527,7 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
        counts + fault word, direction checkpoints, frame, hit records, tile
        claim order, tile times, counters, depth-loop state */
     const size_t o_scene = round256(sizeof(KReq)), o_rows = o_scene + round256(sizeof(StDScene));
-    const size_t o_segs = o_rows + round256((size_t)height1 * 16);
-    const size_t o_rects = o_segs + round256(2 * sizeof(KSeg)), up_host = o_rects;
+    const size_t o_rects = o_rows + round256((size_t)height1 * 16), up_host = o_rects;
     size_t off = o_rects + round256(((size_t)P + 1) * 16);
     auto take = [&](size_t bytes) {
         const size_t o = off;
@@ -2639,8 +2576,10 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
     dv.row_starts = (const float *)(base + o_rows);
     dv.rects = (const int32_t *)(base + o_rects);
     dv.dir_marks = (float *)(base + o_dirs);
-    dv.pixels = base + o_pix;
-    dv.hits = hits ? base + o_hits : NULL;
+    const bool own_px = deliverable(pixels, px * 24, GRID_ALIGN);
+    const bool own_hits = hits && deliverable(hits, px * 16, HITS_ALIGN);
+    dv.pixels = own_px ? (void *)pixels : base + o_pix;
+    dv.hits = !hits ? NULL : own_hits ? (void *)hits : base + o_hits;
     unsigned long long *cnt_d = (unsigned long long *)(base + o_cnt);
     dv.counters = cnt_d;
     rq->row_base = 0;
@@ -2693,15 +2632,6 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
         if (tune.blocks_per_cu < 4)
             (void)capped_blocks(reinterpret_cast<const void *>(k_primary), lds, tune.blocks_per_cu, &lds_primary);
     }
-    /* page-locked outputs are written by the device itself */
-    const bool own_px = deliverable(pixels, px * 24), own_hits = hits && deliverable(hits, px * 16);
-    uint32_t nseg = 0, seg_blocks = 0;
-    auto deliver = [&](size_t src, void *dst, size_t bytes) {
-        ((KSeg *)(g_noalloc_host + o_segs))[nseg++] = KSeg{base + src, (char *)dst, bytes, seg_blocks, 0};
-        seg_blocks += (uint32_t)((bytes + SEG_CHUNK - 1) / SEG_CHUNK);
-    };
-    if (own_px) deliver(o_pix, pixels, px * 24);
-    if (own_hits) deliver(o_hits, hits, px * 16);
     const KReq *reqs_d = (const KReq *)base;
     const StDScene *sc_d = (const StDScene *)(base + o_scene);
     uint32_t *ctr = (uint32_t *)(base + o_ctr);
@@ -2733,11 +2663,7 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
         hipLaunchKernelGGL(k_counts, dim3((tiles + COUNT_TILES - 1) / COUNT_TILES), dim3(256), 0, stream, reqs_d, 1u,
                            (const uint32_t *)w.counts);
     HIP_TRY(hipGetLastError());
-    KDeliver d = {};
-    d.segs = (const KSeg *)(base + o_segs);
-    d.nseg = nseg;
-    d.seg_blocks = seg_blocks;
-    hipLaunchKernelGGL(k_deliver, dim3(seg_blocks + 1), dim3(DELIVER_THREADS), 0, stream, reqs_d, 1u, d,
+    hipLaunchKernelGGL(k_deliver, dim3(1), dim3(DELIVER_THREADS), 0, stream, reqs_d, 1u, KDeliver{},
                        (const unsigned long long *)cnt_d,
                        (unsigned long long *)(g_noalloc_host_dev + ST_NOALLOC_COUNTS), 5u);
     HIP_TRY(hipGetLastError());
