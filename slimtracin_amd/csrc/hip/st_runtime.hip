@@ -888,18 +888,28 @@ __device__ static inline __attribute__((always_inline)) void drain_queue(const K
    back_first 0 takes the refracting pixels (the queue's front part) first,
    1 the others (its back part; on the headline batch the reflecting
    pixels' chains are the long ones: 4.9 against 5.3 ms). */
-/* Queue entries per chunk: 64, or fewer (a power of two, at least this) when
-   there are not enough entries to give every resident wave a chunk of 64.
-   The lanes of a chunk go different ways and wait for each other at every
-   primitive, so a short queue ends sooner spread over idle waves: 9,400
-   pixels of a 1280x720 frame of 64 instances, on 2,048 waves: 2.10 ms in
-   chunks of 64, 1.67 of 16 (at least), 1.58 of 4, 1.61 of 1; queues of 64 and
-   more per wave are cut as before. */
-#define BOUNCE_MIN_WIDTH 4u
+/* Queue entries per chunk: 64, or fewer (a power of two, at least min_width)
+   when there are not enough entries to give every resident wave a chunk of
+   64. The lanes of a chunk go different ways and wait for each other, at
+   every primitive and on every level of a tree, so a short queue ends sooner
+   spread over idle waves; but each of those fetches code, primitives and
+   nodes anew. Stage times with chunks of at least 64, 16 and 4:
+     25 instances, 320x200: 0.71, 0.53, 0.43 ms; 64 instances, 1280x720
+       (9,400 pixels): 2.10, 1.67, 1.58 (of at least 1: 1.61)
+     one mesh of 450,000 triangles, 320x200: 0.66, 0.57, 0.62; 72,000: 0.55,
+       0.46, 0.50; 18,000, 1000x500: 0.42, 0.39, 0.37
+     one mesh of 320 triangles, 320x200: 0.23, 0.23, 0.31; 160x120: 0.24,
+       0.27, 0.28; 4,500, 160x120: 0.34, 0.36, 0.37
+   hence bounce_width: 4 with several primitives, otherwise 16 for large
+   meshes and 64 for small ones; a launch takes the least of its scenes'. */
+static uint32_t bounce_width(const StScene *sc) {
+    return sc->prim_count >= 8u ? 4u : sc->tri_total >= 16384u ? 16u : 64u;
+}
 __global__ void __launch_bounds__(BLOCK_THREADS) K_BOUNCE_ATTR k_bounce(const StDScene *__restrict__ scenes,
                                                           const KReq *__restrict__ reqs, uint32_t nreq, KWave w,
                                                           uint32_t *claim, uint32_t scene_entries,
-                                                          uint32_t mesh_entries, uint32_t back_first) {
+                                                          uint32_t mesh_entries, uint32_t back_first,
+                                                          uint32_t min_width) {
     ST_LDS_STACKS(scene_entries, mesh_entries);
     const DStacks stk = {scene_stack, mesh_stack, nullptr};
     /* the queue's front part (ctr[0] entries) and its back part (ctr[1]
@@ -907,7 +917,7 @@ __global__ void __launch_bounds__(BLOCK_THREADS) K_BOUNCE_ATTR k_bounce(const St
     const uint32_t n_front = __builtin_amdgcn_readfirstlane(ldgu(w.ctr, 0));
     const uint32_t n_back = __builtin_amdgcn_readfirstlane(ldgu(w.ctr, 1));
     uint32_t width = 64u;
-    while (width > BOUNCE_MIN_WIDTH && (n_front + n_back) / (width / 2u) < gridDim.x * WAVES_PER_BLOCK) width >>= 1;
+    while (width > min_width && (n_front + n_back) / (width / 2u) < gridDim.x * WAVES_PER_BLOCK) width >>= 1;
     const uint32_t c_front = (n_front + width - 1u) / width, c_back = (n_back + width - 1u) / width;
     const uint32_t c_first = back_first ? c_back : c_front;
     const uint32_t chunks = w.sorted_q ? (n_front + n_back + width - 1u) / width : c_front + c_back;
@@ -2000,9 +2010,10 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
     }
     /* wavefront buffers of the Beauty depth loop: levels = largest depth,
        shadow planes = largest light count among Beauty requests */
-    uint32_t levels = 0, lmax = 1;
+    uint32_t levels = 0, lmax = 1, min_width = 64;
     for (uint32_t i = 0; i < n; i++)
         if (hv[i].dv.mode == ST_MODE_BEAUTY && hv[i].dv.depth) {
+            if (hv[i].dv.depth > 1) min_width = std::min(min_width, bounce_width(scenes[i]->host));
             if (hv[i].dv.depth > levels) levels = hv[i].dv.depth;
             if (scenes[i]->host->light_count > lmax) lmax = scenes[i]->host->light_count;
         }
@@ -2282,7 +2293,7 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
             }
             hipLaunchKernelGGL(k_bounce, dim3(b_bounce), dim3(BLOCK_THREADS), lds, c->stream,
                                (const StDScene *)sc_d, (const KReq *)reqs_d, n, w, c->tile_counter + BOUNCE_CLAIM,
-                               ks, km, tune.bounce_order);
+                               ks, km, tune.bounce_order, min_width);
             HIP_TRY(mark());
         }
         /* the pixels that gave up, traced again (it reads the queue's length
@@ -2306,7 +2317,7 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
            graph does exactly this launch's work (the per-frame data is in
            the upload block, copied from the same pinned staging) */
         std::vector<uint64_t> sig = {n, up, rows, tiles, levels, lmax, count_blocks, blocks, xcd_blocks, any_device_ssb,
-                                     (uint64_t)claim_mode, s_entries, m_entries, ks, km, (uint64_t)waves4, b_bounce, tune.bounce_order,
+                                     (uint64_t)claim_mode, s_entries, m_entries, ks, km, (uint64_t)waves4, b_bounce, tune.bounce_order, min_width,
                                      lds_primary, (uint64_t)(uintptr_t)blk,
                                      (uint64_t)(uintptr_t)st,
                                      (uint64_t)(uintptr_t)cnt_d, (uint64_t)(uintptr_t)w.st, w.n,
@@ -2655,7 +2666,7 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
     if (beauty && dv.depth > 1) {
         const uint32_t b_bounce = resident_blocks(reinterpret_cast<const void *>(k_bounce), lds);
         hipLaunchKernelGGL(k_bounce, dim3(b_bounce), dim3(BLOCK_THREADS), lds, stream, sc_d, reqs_d, 1u, w,
-                           ctr + BOUNCE_CLAIM, ks, km, tune.bounce_order);
+                           ctr + BOUNCE_CLAIM, ks, km, tune.bounce_order, bounce_width(scene->host));
     }
     hipLaunchKernelGGL(k_redo, dim3(redo_blocks), dim3(redo_threads), lds_redo, stream, sc_d, reqs_d, 1u, w,
                        s_entries, m_entries, coop);
