@@ -2851,9 +2851,11 @@ extern "C" int st_pick(StSceneHandle *scene, const StView *view, uint32_t n, con
     rq->v.rects = (const int32_t *)(blk + o_rect);
     StDScene dsc = scene->dev;
     dsc.fault = NULL;
-    dsc.step_cap = g.step_cap;
-    /* picking traces sequentially: its mesh traversals stop (a fault) at the
-       bound no valid tree reaches, the largest mesh's node count */
+    launch_limits(dsc, g.step_cap, 0, 0);
+    /* picking traces sequentially and has no redo stage: no traversal gives up
+       early (coop_min_tris: not on degenerate rays either); it stops (a fault)
+       at the bound no valid tree reaches, the largest mesh's node count */
+    dsc.coop_min_tris = ~0u;
     uint32_t max_tris = 0;
     for (uint32_t m = 0; m < scene->host->mesh_count; m++)
         if (scene->host->meshes[m].triangle_count > max_tris) max_tris = scene->host->meshes[m].triangle_count;

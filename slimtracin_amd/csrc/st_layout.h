@@ -111,7 +111,9 @@ typedef struct StDScene {
     uint32_t main_step_limit;      /* per launch: mesh traversals of the main stages give up after this
                                       many steps and their pixel is redone (ST_ABANDON_STEPS) */
     uint32_t coop_min_tris;        /* per launch: the redo stage splits traversals of meshes of at least
-                                      this many triangles across a group of blocks (ST_COOP_MIN_TRIS) */
+                                      this many triangles across a group of blocks (ST_COOP_MIN_TRIS), and
+                                      the main stages give degenerate rays on them up early
+                                      (ST_ABANDON_DEGENERATE); all ones in a launch that redoes nothing */
     uint32_t stack_mask_s, stack_mask_m; /* per launch: LDS slots of the scene / mesh traversal stack - 1
                                       (a power of two less one; all ones: the whole stack is in LDS) */
     uint32_t *spill;               /* per launch, with a window: the stacks' older entries, per wave of a
