@@ -1928,6 +1928,17 @@ static uint64_t sig_hash(const std::vector<uint64_t> &w) {
     return h ? h : 1;
 }
 
+/* The library's switches as a launch found them when it began: read once,
+   under the lock, since others may set them while a server's launch runs. */
+struct Switches {
+    StTuning tune;
+    uint32_t step_cap, abandon_steps, coop_min_tris;
+};
+static Switches switches_now(void) {
+    RT_LOCK;
+    return Switches{g.tune, g.step_cap, g.abandon_steps, g.coop_min_tris};
+}
+
 /* Upload and run one launch on context c over `n` requests whose host views
    are already prepared (camera basis, row starts, SSB rects). Each
    request's frame (and hit records) is copied to pixels_host[i] /
@@ -1935,21 +1946,13 @@ static uint64_t sig_hash(const std::vector<uint64_t> &w) {
    the library lock on a server context: only c's own buffers are written,
    the scenes are read. The first `plain` requests have no bounce stage and are
    delivered early (KEarly). */
-static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv, uint32_t n, uint32_t plain,
-                          int want_hits, int persistent, StRayCounts *counts, StFloatPixel *const *pixels_host,
-                          StHitRec *const *hits_host, uint32_t *const *bgra_host, float *kernel_ms) {
-    int rc = ensure_init();
-    if (rc) return rc;
+static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const *scenes, StHostView *hv, uint32_t n,
+                          uint32_t plain, int want_hits, int persistent, StRayCounts *counts,
+                          StFloatPixel *const *pixels_host, StHitRec *const *hits_host, uint32_t *const *bgra_host,
+                          float *kernel_ms) {
+    int rc = ST_OK;
     if (n == 0) return set_err(ST_ERR_ARG, "no requests");
-    StTuning tune;
-    uint32_t step_cap, abandon_steps, coop_min_tris;
-    {
-        RT_LOCK;
-        tune = g.tune;
-        step_cap = g.step_cap;
-        abandon_steps = g.abandon_steps;
-        coop_min_tris = g.coop_min_tris;
-    }
+    const StTuning &tune = sw.tune;
     std::vector<uint32_t> scene_idx(n);
     std::vector<StSceneHandle *> uniq(n);
     uint32_t nuniq = 0;
@@ -2081,9 +2084,10 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
         c->tile_cap = tiles;
     }
     /* the previous launch on this context had this shape: order the tiles
-       by its tile times (when the tuning asks for it) */
-    const uint32_t use_history = (c->tile_sig == tile_sig && g.tune.cost_order == 1u) ? 1u : 0u;
-    const uint32_t order_mode = use_history ? ORDER_HISTORY : g.tune.cost_order == 2u ? ORDER_SUPER : ORDER_TILE;
+       by its tile times (when the tuning asks for it; a launch that is split
+       takes its plain requests' tiles first) */
+    const uint32_t use_history = (!plain && c->tile_sig == tile_sig && tune.cost_order == 1u) ? 1u : 0u;
+    const uint32_t order_mode = use_history ? ORDER_HISTORY : tune.cost_order == 2u ? ORDER_SUPER : ORDER_TILE;
     char *st = c->staging;
     char *blk = (char *)arena_take(&c->work, up);
     KReq *reqs_h = (KReq *)st;
@@ -2097,7 +2101,7 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
     for (uint32_t k = 0; k < nuniq; k++) {
         sc_h[k] = uniq[k]->dev;
         sc_h[k].fault = (uint32_t *)(cnt_d + 3 * (size_t)n);
-        launch_limits(sc_h[k], step_cap, abandon_steps, coop_min_tris, mask_s, mask_m);
+        launch_limits(sc_h[k], sw.step_cap, sw.abandon_steps, sw.coop_min_tris, mask_s, mask_m);
         sc_h[k].spill_s = spill_s;
         sc_h[k].spill_m = spill_m;
     }
@@ -2414,18 +2418,14 @@ static int launch_ordered(LaunchCtx *c, StSceneHandle *const *scenes, StHostView
 int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv, uint32_t n, int want_hits,
                      int persistent, StRayCounts *counts, StFloatPixel *const *pixels_host,
                      StHitRec *const *hits_host, uint32_t *const *bgra_host, float *kernel_ms) {
-    auto straight = [&]() {
-        return launch_ordered(c, scenes, hv, n, 0, want_hits, persistent, counts, pixels_host, hits_host, bgra_host,
-                              kernel_ms);
-    };
     int rc = ensure_init();
     if (rc) return rc;
-    uint32_t cost_order;
-    {
-        RT_LOCK;
-        cost_order = g.tune.cost_order;
-    }
-    if (n < 2 || !persistent || c->graph_mode || cost_order == 1u) return straight();
+    const Switches sw = switches_now();
+    auto straight = [&]() {
+        return launch_ordered(c, sw, scenes, hv, n, 0, want_hits, persistent, counts, pixels_host, hits_host,
+                              bgra_host, kernel_ms);
+    };
+    if (n < 2 || !persistent || c->graph_mode || sw.tune.cost_order == 1u) return straight();
     auto shaded = [&](uint32_t i) { return hv[i].dv.mode == ST_MODE_BEAUTY && hv[i].dv.depth > 1; };
     uint64_t out = 0, px_shaded = 0;
     for (uint32_t i = 0; i < n; i++) {
@@ -2460,7 +2460,7 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
         if (hits_host) o_hits[i] = hits_host[at[i]];
         if (bgra_host) o_bgra[i] = bgra_host[at[i]];
     }
-    rc = launch_ordered(c, o_scenes.data(), o_hv.data(), n, plain, want_hits, persistent,
+    rc = launch_ordered(c, sw, o_scenes.data(), o_hv.data(), n, plain, want_hits, persistent,
                         counts ? o_counts.data() : NULL, pixels_host ? o_px.data() : NULL,
                         hits_host ? o_hits.data() : NULL, bgra_host ? o_bgra.data() : NULL, kernel_ms);
     for (uint32_t i = 0; i < n; i++) {

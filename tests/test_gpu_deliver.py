@@ -5,12 +5,14 @@ as they are."""
 from __future__ import annotations
 
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
 
 import slimtracin_amd as st
 from slimtracin_amd.scene import HIT_DTYPE, MODE_BEAUTY, MODE_DEPTH, MODE_NORMALS, MODE_UVS, PIXEL_DTYPE, make_view
+from slimtracin_amd.server import OUTPUT_BGRA8, Server
 
 pytestmark = pytest.mark.gpu
 
@@ -146,4 +148,41 @@ def test_plain_requests_of_a_mixed_launch(call, abandon):
         assert not abandon or redone
     finally:
         st.debug_redo(0, 0)
+        ds.close()
+
+
+def test_mixed_launches_on_two_contexts_while_the_tuning_changes():
+    """A server's launches of plain and Beauty requests, split and not, two at a time, while another thread sets the
+    claim order: every image equals the one that a launch of its own gives."""
+    ds = st.DeviceScene(st.gen_pbr(3, 30), mesh_lbvh=True)
+    cam = dict(position=(0.0, 3.0, -9.0), pitch=-0.1)
+    kinds = [(2049, 1601, MODE_NORMALS), (1601, 901, MODE_BEAUTY), (2049, 1601, MODE_DEPTH), (1601, 901, MODE_BEAUTY)]
+    views = np.concatenate([make_view(width=w, height=h, mode=m, depth=2, **cam) for w, h, m in kinds])
+    want = [st.render_batch_bgra8([ds], views[i:i + 1])[0][0] for i in range(len(views))]
+    tuned = st.get_tuning()
+    srv = Server(output=OUTPUT_BGRA8, max_in_flight=2, max_batch_requests=16)
+    done = threading.Event()
+
+    def retune():
+        other = st.get_tuning()
+        while not done.is_set():
+            other.cost_order = 1 - other.cost_order
+            st.restore_tuning(other)
+            done.wait(0.0003)
+
+    th = threading.Thread(target=retune)
+    try:
+        sid = srv.add_scene(st.gen_pbr(3, 30), mesh_lbvh=True)
+        th.start()
+        tickets = [srv.submit(sid, views[i % 4:i % 4 + 1]) for i in range(64)]
+        for i, t in enumerate(tickets):
+            image, _, _ = srv.wait(t, timeout_ms=60000)
+            srv.release(t)
+            assert np.array_equal(image, want[i % 4]), i
+    finally:
+        done.set()
+        if th.ident:
+            th.join()
+        st.restore_tuning(tuned)
+        srv.close()
         ds.close()

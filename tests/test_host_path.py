@@ -1,0 +1,106 @@
+"""The library's host path on the CPU: what it queues, copies and waits for, in which order, over a HIP runtime that
+runs no kernels (fake_hip.cpp). Each case runs in a process of its own, with that runtime in place of the real one."""
+from __future__ import annotations
+
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CASES = {}
+
+
+def case(f):
+    CASES[f.__name__] = f
+    return f
+
+
+class Fake:
+    """The runtime, loaded before the library, and a log of its calls; act(name, args) runs at each of them."""
+
+    def __init__(self, so):
+        self.so = C.CDLL(so, mode=C.RTLD_GLOBAL)
+        self.so.fake_device_bytes.restype = C.c_size_t
+        self.so.fake_host_alloc.restype = C.c_void_p
+        self.log, self.act = [], None
+        self.hook = C.CFUNCTYPE(None, C.c_char_p, C.POINTER(C.c_void_p))(self._call)
+        self.so.fake_hook(self.hook)
+
+    def _call(self, name, args):
+        name = name.decode()
+        if name.startswith("launch _Z"):   # the kernel's plain name
+            digits = "".join(c for c in name[9:12] if c.isdigit())
+            name = "launch " + name[9 + len(digits):][:int(digits)]
+        self.log.append(name)
+        if self.act:
+            self.act(name, args)
+
+    def u32(self, args, i):
+        return C.cast(args[i], C.POINTER(C.c_uint32))[0]
+
+
+def _mixed_batch(st):
+    """Requests without a bounce stage with 62 MB of window images and 6 million pixels that have one: a launch that
+    is split, the former delivered while the latter render."""
+    import numpy as np
+    from slimtracin_amd.scene import MODE_BEAUTY, MODE_NORMALS, make_view
+    ds = st.DeviceScene(st.gen_pbr(3, 30), mesh_binned=True)
+    views = np.concatenate([make_view(width=3839, height=2023, mode=m, depth=3)
+                            for m in (MODE_NORMALS, MODE_BEAUTY, MODE_NORMALS)])
+    outs = st.pinned_split([3839 * 2023] * 3, np.uint32)
+    return [ds] * 3, views, outs
+
+
+@case
+def split_keeps_its_tile_order(fake, st):
+    """A launch that is split has its plain requests' tiles first in the claim order; a tuning with an order of its own
+    that arrives while the launch is being prepared is for the next one."""
+    scenes, views, outs = _mixed_batch(st)
+    st.render_batch_bgra8(scenes, views, outs=outs)
+    modes = []
+    tuned = st.get_tuning()
+
+    def act(name, args):
+        if name.startswith("hipOccupancy"):
+            tuned.cost_order = 1
+            st.restore_tuning(tuned)
+        if name == "launch k_prep":
+            modes.append(fake.u32(args, 10))
+
+    fake.log.clear()
+    fake.act = act
+    st.render_batch_bgra8(scenes, views, outs=outs)
+    assert fake.log.count("launch k_primary4") == 2, fake.log
+    assert modes == [0], modes   # tile order
+    del fake.log[:], modes[:]
+    for _ in range(2):
+        st.render_batch_bgra8(scenes, views, outs=outs)
+    assert fake.log.count("launch k_primary4") == 2, fake.log
+    assert modes == [0, 1], modes   # slowest first, once this order's times are known
+
+
+@pytest.fixture(scope="module")
+def fake_so(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", os.path.join(HERE, "fake_hip.cpp"), "-o", so],
+                   check=True)
+    return so
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_host_path(fake_so, name):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), fake_so, name], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-4000:])
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, os.path.dirname(HERE))
+    runtime = Fake(sys.argv[1])
+    import slimtracin_amd as library
+    library.init(0)
+    CASES[sys.argv[2]](runtime, library)
+    runtime.act = None
