@@ -137,7 +137,8 @@ int st_render(StSceneHandle *scene, const StView *view, StFloatPixel *pixels, St
 int st_render_noalloc(StSceneHandle *scene, const StView *view, StFloatPixel *pixels, StHitRec *hits,
                       StRayCounts *counts);
 
-/* n requests fused into one launch. pixels[i] / hits[i] may be NULL. */
+/* n requests fused into one launch. pixels[i] / hits[i] may be NULL. Where
+   outputs of one call overlap, the last request's stand. */
 int st_render_batch(StSceneHandle *const *scenes, const StView *views, uint32_t n, StFloatPixel *const *pixels,
                     StHitRec *const *hits, StRayCounts *counts, uint32_t flags);
 
@@ -199,8 +200,11 @@ int st_ssb(StSceneHandle *scene, const StView *view, int32_t *rects, uint8_t *fl
    per point. */
 int st_pick(StSceneHandle *scene, const StView *view, uint32_t n, const uint32_t *xy, StPick *out);
 
-/* Page-locked host memory for frame outputs: downloads into it run at the
-   link's full rate (pageable destinations are staged by the runtime). */
+/* Page-locked host memory for frame outputs. The device writes outputs in it
+   directly (grids aligned to 8 bytes, hit records to 16, window images to 4;
+   others are copied there afterwards), at any time during the call that asks
+   for them and in any order: what was in them before is gone from the call's
+   start on, and a call that fails leaves them undefined. */
 int st_host_alloc(size_t bytes, void **out);
 void st_host_free(void *p);
 

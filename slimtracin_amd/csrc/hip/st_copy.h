@@ -65,12 +65,14 @@ static inline bool words_below(const char *p, size_t bytes, uint32_t limit) {
 
 /* Copy the spans between pageable host memory and the device on `stream`,
    after the work queued there; complete when the call returns. Plain copy
-   calls where the whole is small or the ring or its threads cannot be had.
+   calls where the whole is small or the ring or its threads cannot be had,
+   and where the spans have to be copied one after another (in_order: they
+   overlap).
    *in_range (uploads) tells whether all indices are below their limits: the
    threads look while they have the bytes at hand (24 MB of indices by
    themselves, on one thread: 2 ms). */
 static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const std::vector<CopySpan> &spans,
-                                       bool download, bool *in_range = nullptr) {
+                                       bool download, bool in_order, bool *in_range = nullptr) {
     size_t total = 0;
     for (const CopySpan &s : spans) total += s.bytes;
     std::atomic<uint32_t> over(0);
@@ -85,7 +87,7 @@ static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const
         return e != hipSuccess ? e : hipStreamSynchronize(stream);
     };
     if (in_range) *in_range = true;
-    if (total < COPY_MIN_BYTES || !copy_ring_ready(ring)) return plain();
+    if (in_order || total < COPY_MIN_BYTES || !copy_ring_ready(ring)) return plain();
     std::vector<CopySpan> chunk;
     chunk.reserve(total / COPY_SLOT_BYTES + spans.size());
     for (const CopySpan &s : spans)

@@ -1575,7 +1575,7 @@ static int build_device_meshes(StSceneHandle *h) {
             rc = set_err(ST_ERR_SCENE, "invalid scene: mesh index out of range");
             break;
         }
-        if (copy_pageable(g.main.stream, &g.main.ring, spans, false, &in_range) != hipSuccess) {
+        if (copy_pageable(g.main.stream, &g.main.ring, spans, false, false, &in_range) != hipSuccess) {
             rc = set_err(ST_ERR_HIP, "mesh geometry upload failed");
             break;
         }
@@ -1698,7 +1698,7 @@ extern "C" int st_scene_upload(StSceneHandle *h) {
     std::vector<CopySpan> spans;
     for (size_t i = 0; i < sizeof parts / sizeof parts[0]; i++)
         if (parts[i].bytes) spans.push_back({b + parts[i].off, (char *)parts[i].src, parts[i].bytes, 0});
-    HIP_TRY(copy_pageable(g.main.stream, &g.main.ring, spans, false));
+    HIP_TRY(copy_pageable(g.main.stream, &g.main.ring, spans, false, false));
     if (sc->mesh_count) {
         float *ma = (float *)malloc(24ull * sc->mesh_count);
         for (uint32_t m = 0; m < sc->mesh_count; m++) {
@@ -1928,6 +1928,27 @@ static uint64_t sig_hash(const std::vector<uint64_t> &w) {
     return h ? h : 1;
 }
 
+/* Whether two outputs of a launch share memory. Such ones are not written by
+   the device: they are copied one after another in the requests' order, so
+   that the last one stands. */
+static bool outputs_overlap(const StHostView *hv, uint32_t n, int want_hits, StFloatPixel *const *pixels_host,
+                            StHitRec *const *hits_host, uint32_t *const *bgra_host) {
+    std::vector<std::pair<uintptr_t, uintptr_t>> spans;
+    auto add = [&](const void *p, uint64_t bytes) {
+        if (p) spans.push_back({(uintptr_t)p, (uintptr_t)p + bytes});
+    };
+    for (uint32_t i = 0; i < n; i++) {
+        const uint64_t w1 = hv[i].dv.width1, h1 = hv[i].dv.height1;
+        if (pixels_host) add(pixels_host[i], w1 * h1 * 24);
+        if (want_hits && hits_host) add(hits_host[i], w1 * h1 * 16);
+        if (bgra_host && w1 > 1 && h1 > 1) add(bgra_host[i], (w1 - 1) * (h1 - 1) * 4);
+    }
+    std::sort(spans.begin(), spans.end());
+    for (size_t k = 1; k < spans.size(); k++)
+        if (spans[k].first < spans[k - 1].second) return true;
+    return false;
+}
+
 /* The library's switches as a launch found them when it began: read once,
    under the lock, since others may set them while a server's launch runs. */
 struct Switches {
@@ -1945,9 +1966,9 @@ static Switches switches_now(void) {
    hits_host[i] when given. Returns when the launch is done. Runs without
    the library lock on a server context: only c's own buffers are written,
    the scenes are read. The first `plain` requests have no bounce stage and are
-   delivered early (KEarly). */
+   delivered early (KEarly). apart: no two outputs overlap. */
 static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const *scenes, StHostView *hv, uint32_t n,
-                          uint32_t plain, int want_hits, int persistent, StRayCounts *counts,
+                          uint32_t plain, bool apart, int want_hits, int persistent, StRayCounts *counts,
                           StFloatPixel *const *pixels_host, StHitRec *const *hits_host, uint32_t *const *bgra_host,
                           float *kernel_ms) {
     int rc = ST_OK;
@@ -1980,13 +2001,13 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
         if (bgra_host && bgra_host[i]) {
             if (hv[i].dv.width1 < 2 || hv[i].dv.height1 < 2) return set_err(ST_ERR_ARG, "request %u: empty window", i);
             const size_t wb = (size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4;
-            own_bgra[i] = deliverable(bgra_host[i], wb, IMAGE_ALIGN);
+            own_bgra[i] = apart && deliverable(bgra_host[i], wb, IMAGE_ALIGN);
             if (!own_bgra[i]) per_req_out += round256(wb);
         }
         /* (the resolve reads the grid: it stays in device memory) */
-        own_px[i] = pixels_host && pixels_host[i] && !(bgra_host && bgra_host[i]) &&
+        own_px[i] = apart && pixels_host && pixels_host[i] && !(bgra_host && bgra_host[i]) &&
                     deliverable(pixels_host[i], px * 24, GRID_ALIGN);
-        own_hits[i] = want_hits && hits_host && hits_host[i] && deliverable(hits_host[i], px * 16, HITS_ALIGN);
+        own_hits[i] = apart && want_hits && hits_host && hits_host[i] && deliverable(hits_host[i], px * 16, HITS_ALIGN);
         if (!own_px[i]) per_req_out += round256(px * 24);
         if (want_hits && !own_hits[i]) per_req_out += round256(px * 16);
         const uint32_t tw = 1u << tune.tile_shift, th = 64u >> tune.tile_shift;
@@ -2390,7 +2411,7 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
             spans.push_back({(char *)reqs_h[i].bgra, (char *)bgra_host[i],
                              (size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4, 0});
     }
-    if (!spans.empty()) HIP_TRY(copy_pageable(c->stream, &c->ring, spans, true));
+    if (!spans.empty()) HIP_TRY(copy_pageable(c->stream, &c->ring, spans, true, !apart));
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->last_redo = (uint32_t)cnt_h[3 * (size_t)n + 1];
     if (cnt_h[3 * (size_t)n])
@@ -2421,11 +2442,12 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
     int rc = ensure_init();
     if (rc) return rc;
     const Switches sw = switches_now();
+    const bool apart = !outputs_overlap(hv, n, want_hits, pixels_host, hits_host, bgra_host);
     auto straight = [&]() {
-        return launch_ordered(c, sw, scenes, hv, n, 0, want_hits, persistent, counts, pixels_host, hits_host,
+        return launch_ordered(c, sw, scenes, hv, n, 0, apart, want_hits, persistent, counts, pixels_host, hits_host,
                               bgra_host, kernel_ms);
     };
-    if (n < 2 || !persistent || c->graph_mode || sw.tune.cost_order == 1u) return straight();
+    if (n < 2 || !apart || !persistent || c->graph_mode || sw.tune.cost_order == 1u) return straight();
     auto shaded = [&](uint32_t i) { return hv[i].dv.mode == ST_MODE_BEAUTY && hv[i].dv.depth > 1; };
     uint64_t out = 0, px_shaded = 0;
     for (uint32_t i = 0; i < n; i++) {
@@ -2460,7 +2482,7 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
         if (hits_host) o_hits[i] = hits_host[at[i]];
         if (bgra_host) o_bgra[i] = bgra_host[at[i]];
     }
-    rc = launch_ordered(c, sw, o_scenes.data(), o_hv.data(), n, plain, want_hits, persistent,
+    rc = launch_ordered(c, sw, o_scenes.data(), o_hv.data(), n, plain, true, want_hits, persistent,
                         counts ? o_counts.data() : NULL, pixels_host ? o_px.data() : NULL,
                         hits_host ? o_hits.data() : NULL, bgra_host ? o_bgra.data() : NULL, kernel_ms);
     for (uint32_t i = 0; i < n; i++) {
@@ -2587,8 +2609,10 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
     dv.row_starts = (const float *)(base + o_rows);
     dv.rects = (const int32_t *)(base + o_rects);
     dv.dir_marks = (float *)(base + o_dirs);
-    const bool own_px = deliverable(pixels, px * 24, GRID_ALIGN);
-    const bool own_hits = hits && deliverable(hits, px * 16, HITS_ALIGN);
+    const bool apart = !hits || (uintptr_t)hits >= (uintptr_t)pixels + px * 24 ||
+                       (uintptr_t)pixels >= (uintptr_t)hits + px * 16;
+    const bool own_px = apart && deliverable(pixels, px * 24, GRID_ALIGN);
+    const bool own_hits = apart && hits && deliverable(hits, px * 16, HITS_ALIGN);
     dv.pixels = own_px ? (void *)pixels : base + o_pix;
     dv.hits = !hits ? NULL : own_hits ? (void *)hits : base + o_hits;
     unsigned long long *cnt_d = (unsigned long long *)(base + o_cnt);

@@ -186,3 +186,23 @@ def test_mixed_launches_on_two_contexts_while_the_tuning_changes():
         st.restore_tuning(tuned)
         srv.close()
         ds.close()
+
+
+@pytest.mark.parametrize("kind", ["page-locked", "pageable"])
+@pytest.mark.parametrize("shift", [0, 1, 40001])
+def test_outputs_that_share_memory(scene, kind, shift):
+    """Of outputs that overlap the last request's stands, as if the requests had been rendered one after another."""
+    w, h, cam = 320, 250, dict(position=(0.0, 7.0, -11.0), pitch=-0.2)
+    n = (w + 1) * (h + 1)
+    views = np.concatenate([make_view(width=w, height=h, mode=m, depth=2, **cam)
+                            for m in (MODE_BEAUTY, MODE_DEPTH, MODE_NORMALS)])
+    size = n + 2 * shift
+    for dtype, pixels, call in ((PIXEL_DTYPE, n, st.render_batch), (np.uint32, w * h, st.render_batch_bgra8)):
+        block = st.pinned_empty(size, dtype) if kind == "page-locked" else np.zeros(size, dtype)
+        block.view(np.uint8)[:] = 0
+        want = block.copy()
+        alone = [call([scene], views[i:i + 1])[0][0] for i in range(3)]
+        for i in range(3):
+            want[i * shift:i * shift + pixels] = alone[i]
+        call([scene] * 3, views, outs=[block[i * shift:i * shift + pixels] for i in range(3)])
+        assert block.tobytes() == want.tobytes()

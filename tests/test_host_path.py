@@ -82,6 +82,34 @@ def split_keeps_its_tile_order(fake, st):
     assert modes == [0, 1], modes   # slowest first, once this order's times are known
 
 
+@case
+def outputs_that_share_memory_are_copied_in_order(fake, st):
+    """Nobody writes such outputs directly, nor with several threads: one copy after another, in the requests' order."""
+    import numpy as np
+    from slimtracin_amd.scene import MODE_BEAUTY, MODE_DEPTH, PIXEL_DTYPE, make_view
+    ds = st.DeviceScene(st.gen_implicit(3))
+    w, h = 599, 499
+    views = np.concatenate([make_view(width=w, height=h, mode=m, depth=2) for m in (MODE_DEPTH, MODE_BEAUTY, MODE_DEPTH)])
+    copies = []
+    fake.act = lambda name, args: copies.append((args[0], args[2])) if name == "hipMemcpyAsync" else None
+    n = (w + 1) * (h + 1)
+    for block in (st.pinned_empty(2 * n, PIXEL_DTYPE), np.empty(2 * n, PIXEL_DTYPE)):
+        for outs in ([block[:n], block[n:], block[:n]], [block[:n], block[n // 2:n // 2 + n], block[n:]]):
+            del copies[:]
+            st.render_batch([ds] * 3, views, outs=outs)
+            assert copies == [(o.ctypes.data, 24 * n) for o in outs], copies
+    block = st.pinned_empty(2 * w * h + 1, np.uint32)
+    for outs in ([block[:w * h]] * 3, [block[1:w * h + 1], block[w * h + 1:], block[:w * h]]):
+        del copies[:]
+        st.render_batch_bgra8([ds] * 3, views, outs=outs)
+        assert copies == [(o.ctypes.data, 4 * w * h) for o in outs], copies
+    one = st.pinned_empty(3 * n, PIXEL_DTYPE)
+    one = [one[:n], one[n:2 * n], one[2 * n:]]   # neighbours that do not overlap are written by the device
+    del copies[:]
+    st.render_batch([ds] * 3, views, outs=one)
+    assert not copies, copies
+
+
 @pytest.fixture(scope="module")
 def fake_so(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
