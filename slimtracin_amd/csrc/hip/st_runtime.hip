@@ -67,6 +67,17 @@
 #include "st_sort.h"
 #include "st_copy.h"
 
+/* Waits for a stream at the end of its scope, unless what was queued there
+   has been waited for: a call that fails half way must not return while
+   kernels read its staging or write the caller's outputs. */
+struct StreamGuard {
+    hipStream_t stream;
+    bool pending;
+    ~StreamGuard() {
+        if (pending) (void)hipStreamSynchronize(stream);
+    }
+};
+
 #define WAVES_PER_BLOCK 4
 #define BLOCK_THREADS (64 * WAVES_PER_BLOCK)
 /* Launch attributes of the primary stage (occupancy experiments): 3 waves
@@ -2334,6 +2345,7 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
         return ST_OK;
     };
 
+    StreamGuard guard = {c->stream, true};
     if (!graph) {
         if ((rc = enqueue())) return rc;
     } else {
@@ -2413,6 +2425,7 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
     }
     if (!spans.empty()) HIP_TRY(copy_pageable(c->stream, &c->ring, spans, true, !apart));
     HIP_TRY(hipStreamSynchronize(c->stream));
+    guard.pending = false;
     c->last_redo = (uint32_t)cnt_h[3 * (size_t)n + 1];
     if (cnt_h[3 * (size_t)n])
         return set_err(ST_ERR_SCENE, "a traversal ran past its bound (fault bits 0x%llx): malformed BVH",
@@ -2671,6 +2684,7 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
     const StDScene *sc_d = (const StDScene *)(base + o_scene);
     uint32_t *ctr = (uint32_t *)(base + o_ctr);
     hipStream_t stream = g.main.stream;
+    StreamGuard guard = {stream, true};
     /* the request, scene record and row starts; the rects region is filled
        by the device SSB pass */
     hipLaunchKernelGGL(k_setup, dim3(setup_blocks(up_host)), dim3(SETUP_THREADS), 0, stream,
@@ -2705,6 +2719,7 @@ extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFlo
     if (!own_px) HIP_TRY(hipMemcpyAsync(pixels, base + o_pix, px * 24, hipMemcpyDeviceToHost, stream));
     if (hits && !own_hits) HIP_TRY(hipMemcpyAsync(hits, base + o_hits, px * 16, hipMemcpyDeviceToHost, stream));
     HIP_TRY(hipStreamSynchronize(stream));
+    guard.pending = false;
     const unsigned long long *counts_h = (const unsigned long long *)(g_noalloc_host + ST_NOALLOC_COUNTS);
     if (counts_h[3])
         return set_err(ST_ERR_SCENE, "a traversal ran past its bound (fault bits 0x%llx): malformed BVH",
@@ -2902,6 +2917,7 @@ extern "C" int st_pick(StSceneHandle *scene, const StView *view, uint32_t n, con
     pk.fault = (uint32_t *)(g.main.staging_dev + o_fault);
     st_view_release(&hv);
     const uint32_t m_entries = scene->dev.mesh_stack_size > 1 ? scene->dev.mesh_stack_size : 1;
+    StreamGuard guard = {g.main.stream, true};
     hipLaunchKernelGGL(k_setup, dim3(setup_blocks(up)), dim3(SETUP_THREADS), 0, g.main.stream,
                        (const uint4 *)g.main.staging_dev, (uint4 *)blk, (uint32_t)(up / 16),
                        (unsigned long long *)NULL, 0u, (uint32_t *)NULL, 0u, (uint32_t *)NULL, (uint32_t *)NULL);
@@ -2909,6 +2925,7 @@ extern "C" int st_pick(StSceneHandle *scene, const StView *view, uint32_t n, con
                        (const StDScene *)(blk + o_sc), (const KReq *)blk, pk, m_entries);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(g.main.stream));
+    guard.pending = false;
     const uint32_t fault = *(const uint32_t *)(g.main.staging + o_fault);
     memcpy(out, g.main.staging + o_out, n * sizeof(StPick));
     if (fault) return set_err(ST_ERR_SCENE, "a traversal ran past its bound (fault bits 0x%x): malformed BVH", fault);

@@ -110,6 +110,42 @@ def outputs_that_share_memory_are_copied_in_order(fake, st):
     assert not copies, copies
 
 
+@case
+def a_failed_call_has_waited_for_its_kernels(fake, st):
+    """Whichever call fails after kernels were queued, the stream is waited for before the error is returned."""
+    import numpy as np
+    from slimtracin_amd.scene import MODE_BEAUTY, PIXEL_DTYPE, make_view
+    ds = st.DeviceScene(st.gen_pbr(3, 10))
+    view = make_view(width=90, height=70, mode=MODE_BEAUTY, depth=3)
+    out = st.pinned_empty(91 * 71, PIXEL_DTYPE)
+    xy = np.array([[3, 4], [40, 30]], np.uint32)
+    calls = {"render": lambda: st.render(ds, view), "pinned": lambda: st.render(ds, view, hits=False, out=out),
+             "noalloc": lambda: st.render_noalloc(ds, view, out=out), "pick": lambda: st.pick(ds, view, xy),
+             "graph": lambda: st.render_batch([ds], view, graph=True), "timed": lambda: st.render_timed([ds], view, stages=True),
+             "images": lambda: st.render_batch_bgra8([ds], view)}
+    failed = 0
+    for what, call in calls.items():
+        call()
+        for name in ("hipGetLastError", "hipMemcpyAsync", "hipEventRecord", "hipGraphLaunch", "hipStreamSynchronize",
+                     "hipEventSynchronize"):
+            for nth in range(1, 12):
+                fake.so.fake_fail(name.encode(), nth)
+                del fake.log[:]
+                try:
+                    call()
+                except st.SlimTracinError:
+                    failed += 1
+                    queued = [i for i, c in enumerate(fake.log) if c.startswith("launch ")]
+                    waits = [i for i, c in enumerate(fake.log) if c == "hipStreamSynchronize"]
+                    if queued:
+                        assert waits and waits[-1] > queued[-1], (what, name, nth, fake.log)
+                        assert name != "hipStreamSynchronize" or len(waits) > 1, (what, nth, fake.log)
+                else:
+                    fake.so.fake_fail(b"", 0)
+                    break
+    assert failed > 25, failed
+
+
 @pytest.fixture(scope="module")
 def fake_so(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
