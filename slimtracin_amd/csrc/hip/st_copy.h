@@ -117,12 +117,14 @@ static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const
         }
     };
     std::vector<std::thread> team;
-    try {
-        team.reserve(COPY_THREADS);
-        for (uint32_t t = 0; t < COPY_THREADS && t < chunks; t++) team.emplace_back(work);
-    } catch (const std::system_error &) {
-        if (team.empty()) return plain();
-    }
+    auto start_team = [&]() {
+        try {
+            team.reserve(COPY_THREADS);
+            for (uint32_t t = 0; t < COPY_THREADS && t < chunks; t++) team.emplace_back(work);
+        } catch (const std::system_error &) {
+        }
+        return !team.empty();
+    };
     hipError_t e = hipSuccess;
     auto wait_moved = [&](uint32_t i) {
         while (!moved[i].load(std::memory_order_acquire)) std::this_thread::yield();
@@ -136,6 +138,10 @@ static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const
     };
     if (download) {
         for (uint32_t i = 0; i < chunks && i < COPY_SLOTS && e == hipSuccess; i++) e = queue(i);
+        /* the threads start when there is something to move: the stream may
+           have a whole render ahead of the copies */
+        if (e == hipSuccess) e = hipEventSynchronize(ring->ev[0]);
+        if (e == hipSuccess && !start_team()) return plain();
         for (uint32_t i = 0; i < chunks && e == hipSuccess; i++) {
             e = hipEventSynchronize(ring->ev[i % COPY_SLOTS]);
             if (e != hipSuccess) break;
@@ -148,6 +154,7 @@ static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const
         }
         for (uint32_t i = 0; i < chunks && e == hipSuccess; i++) wait_moved(i);
     } else {
+        if (!start_team()) return plain();
         for (uint32_t i = 0; i < chunks && i < COPY_SLOTS; i++) open[i].store(1, std::memory_order_release);
         for (uint32_t i = 0; i < chunks && e == hipSuccess; i++) {
             wait_moved(i);

@@ -146,6 +146,37 @@ def a_failed_call_has_waited_for_its_kernels(fake, st):
     assert failed > 25, failed
 
 
+def _threads():
+    return len(os.listdir("/proc/self/task"))
+
+
+@case
+def copying_threads_start_when_there_is_something_to_copy(fake, st):
+    """A large download is queued behind the render; its threads start after the first bytes have arrived, and the call
+    takes no processor time of theirs while it waits for the device."""
+    import time
+    import numpy as np
+    from slimtracin_amd.scene import MODE_DEPTH, make_view
+    ds = st.DeviceScene(st.gen_implicit(3))
+    view = make_view(width=1000, height=700, mode=MODE_DEPTH)
+    st.render(ds, view)
+    before, seen = _threads(), []
+
+    def act(name, args):
+        if name in ("hipEventSynchronize", "hipStreamSynchronize"):
+            if not seen:
+                t0 = time.process_time()
+                time.sleep(0.3)   # the device renders
+                seen.append((_threads(), time.process_time() - t0))
+            else:
+                seen.append((_threads(), 0.0))
+
+    fake.act = act
+    st.render(ds, view)
+    assert seen[0][0] == before and seen[0][1] < 1.0, (before, seen[0])
+    assert max(n for n, _ in seen) > before, seen   # the ring was used
+
+
 @pytest.fixture(scope="module")
 def fake_so(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
