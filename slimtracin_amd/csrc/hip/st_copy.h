@@ -15,8 +15,10 @@
 
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
-#include <system_error>
+#include <exception>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -71,14 +73,15 @@ static inline bool words_below(const char *p, size_t bytes, uint32_t limit) {
    *in_range (uploads) tells whether all indices are below their limits: the
    threads look while they have the bytes at hand (24 MB of indices by
    themselves, on one thread: 2 ms). */
-static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const std::vector<CopySpan> &spans,
+static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const CopySpan *spans, size_t nspans,
                                        bool download, bool in_order, bool *in_range = nullptr) {
     size_t total = 0;
-    for (const CopySpan &s : spans) total += s.bytes;
+    for (size_t k = 0; k < nspans; k++) total += spans[k].bytes;
     std::atomic<uint32_t> over(0);
     auto plain = [&]() {
         hipError_t e = hipSuccess;
-        for (const CopySpan &s : spans) {
+        for (size_t k = 0; k < nspans; k++) {
+            const CopySpan &s = spans[k];
             if (!s.bytes || e != hipSuccess) continue;
             if (in_range && s.limit && !words_below(s.host, s.bytes, s.limit)) *in_range = false;
             e = download ? hipMemcpyAsync(s.host, s.dev, s.bytes, hipMemcpyDeviceToHost, stream)
@@ -89,16 +92,24 @@ static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const
     if (in_range) *in_range = true;
     if (in_order || total < COPY_MIN_BYTES || !copy_ring_ready(ring)) return plain();
     std::vector<CopySpan> chunk;
-    chunk.reserve(total / COPY_SLOT_BYTES + spans.size());
-    for (const CopySpan &s : spans)
-        for (size_t at = 0; at < s.bytes; at += COPY_SLOT_BYTES)
-            chunk.push_back({s.dev + at, s.host + at,
-                             s.bytes - at < COPY_SLOT_BYTES ? s.bytes - at : (size_t)COPY_SLOT_BYTES, s.limit});
-    const uint32_t chunks = (uint32_t)chunk.size();
     /* A chunk's state: `open` says that its slot may be moved by a thread (the
        download into it is done, or the upload before it has left it), `moved`
        that a thread has done so. Threads take chunks in order. */
-    std::vector<std::atomic<uint32_t>> open(chunks), moved(chunks);
+    std::vector<std::atomic<uint32_t>> open, moved;
+    std::vector<std::thread> team;
+    try {
+        chunk.reserve(total / COPY_SLOT_BYTES + nspans);
+        for (size_t k = 0; k < nspans; k++)
+            for (size_t at = 0; at < spans[k].bytes; at += COPY_SLOT_BYTES)
+                chunk.push_back({spans[k].dev + at, spans[k].host + at,
+                                 std::min(spans[k].bytes - at, (size_t)COPY_SLOT_BYTES), spans[k].limit});
+        std::vector<std::atomic<uint32_t>>(chunk.size()).swap(open);
+        std::vector<std::atomic<uint32_t>>(chunk.size()).swap(moved);
+        team.reserve(COPY_THREADS);
+    } catch (const std::bad_alloc &) {
+        return plain();
+    }
+    const uint32_t chunks = (uint32_t)chunk.size();
     for (uint32_t i = 0; i < chunks; i++) open[i] = moved[i] = 0;
     std::atomic<uint32_t> next(0), stop(0);
     auto work = [&]() {
@@ -116,12 +127,10 @@ static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const
             moved[i].store(1, std::memory_order_release);
         }
     };
-    std::vector<std::thread> team;
     auto start_team = [&]() {
         try {
-            team.reserve(COPY_THREADS);
             for (uint32_t t = 0; t < COPY_THREADS && t < chunks; t++) team.emplace_back(work);
-        } catch (const std::system_error &) {
+        } catch (const std::exception &) {   /* no thread or no memory for one: those that run do it */
         }
         return !team.empty();
     };

@@ -1574,10 +1574,11 @@ static int build_device_meshes(StSceneHandle *h) {
             {q->uvs_count ? s->uvs : NULL, 8ull * q->uvs_count, (const void **)&in.uvs, 0},
             {q->uvs_count ? s->uidx : NULL, 12ull * q->triangle_count, (const void **)&in.uidx, q->uvs_count},
         };
-        std::vector<CopySpan> spans;
+        CopySpan spans[6];
+        size_t nspans = 0;
         for (int k = 0; k < 6; k++) {
             if (!up[k].src || !up[k].bytes) continue;
-            spans.push_back({p, (char *)up[k].src, up[k].bytes, up[k].limit});
+            spans[nspans++] = {p, (char *)up[k].src, up[k].bytes, up[k].limit};
             *up[k].dst = p;
             p += round256(up[k].bytes);
         }
@@ -1586,7 +1587,7 @@ static int build_device_meshes(StSceneHandle *h) {
             rc = set_err(ST_ERR_SCENE, "invalid scene: mesh index out of range");
             break;
         }
-        if (copy_pageable(g.main.stream, &g.main.ring, spans, false, false, &in_range) != hipSuccess) {
+        if (copy_pageable(g.main.stream, &g.main.ring, spans, nspans, false, false, &in_range) != hipSuccess) {
             rc = set_err(ST_ERR_HIP, "mesh geometry upload failed");
             break;
         }
@@ -1706,10 +1707,11 @@ extern "C" int st_scene_upload(StSceneHandle *h) {
         {o_mips, sc->mips, sc->mip_total * sizeof(StDMip)},
         {o_texels, sc->texels, sc->texel_bytes},
     };
-    std::vector<CopySpan> spans;
+    CopySpan spans[sizeof parts / sizeof parts[0]];
+    size_t nspans = 0;
     for (size_t i = 0; i < sizeof parts / sizeof parts[0]; i++)
-        if (parts[i].bytes) spans.push_back({b + parts[i].off, (char *)parts[i].src, parts[i].bytes, 0});
-    HIP_TRY(copy_pageable(g.main.stream, &g.main.ring, spans, false, false));
+        if (parts[i].bytes) spans[nspans++] = {b + parts[i].off, (char *)parts[i].src, parts[i].bytes, 0};
+    HIP_TRY(copy_pageable(g.main.stream, &g.main.ring, spans, nspans, false, false));
     if (sc->mesh_count) {
         float *ma = (float *)malloc(24ull * sc->mesh_count);
         for (uint32_t m = 0; m < sc->mesh_count; m++) {
@@ -2423,7 +2425,7 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
             spans.push_back({(char *)reqs_h[i].bgra, (char *)bgra_host[i],
                              (size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4, 0});
     }
-    if (!spans.empty()) HIP_TRY(copy_pageable(c->stream, &c->ring, spans, true, !apart));
+    if (!spans.empty()) HIP_TRY(copy_pageable(c->stream, &c->ring, spans.data(), spans.size(), true, !apart));
     HIP_TRY(hipStreamSynchronize(c->stream));
     guard.pending = false;
     c->last_redo = (uint32_t)cnt_h[3 * (size_t)n + 1];
@@ -2449,9 +2451,9 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
    captured graph keeps its outputs out of the graph, so its launches are not
    split; neither are those with an order of tiles of their own
    (StTuning.cost_order 1) or one wave per tile. */
-int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv, uint32_t n, int want_hits,
-                     int persistent, StRayCounts *counts, StFloatPixel *const *pixels_host,
-                     StHitRec *const *hits_host, uint32_t *const *bgra_host, float *kernel_ms) {
+static int launch_split(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv, uint32_t n, int want_hits,
+                        int persistent, StRayCounts *counts, StFloatPixel *const *pixels_host,
+                        StHitRec *const *hits_host, uint32_t *const *bgra_host, float *kernel_ms) {
     int rc = ensure_init();
     if (rc) return rc;
     const Switches sw = switches_now();
@@ -2503,6 +2505,19 @@ int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv,
         if (counts) counts[at[i]] = o_counts[i];
     }
     return rc;
+}
+
+/* A launch's host arrays are C++ ones: running out of memory for them is an
+   error like any other to the C callers and the server's workers. */
+int st_rt_launch_ctx(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *hv, uint32_t n, int want_hits,
+                     int persistent, StRayCounts *counts, StFloatPixel *const *pixels_host,
+                     StHitRec *const *hits_host, uint32_t *const *bgra_host, float *kernel_ms) {
+    try {
+        return launch_split(c, scenes, hv, n, want_hits, persistent, counts, pixels_host, hits_host, bgra_host,
+                            kernel_ms);
+    } catch (const std::bad_alloc &) {
+        return set_err(ST_ERR_MEMORY, "out of host memory");
+    }
 }
 
 int st_rt_launch_prepared(StSceneHandle *const *scenes, StHostView *hv, uint32_t n, int want_hits, int persistent,
@@ -2972,7 +2987,13 @@ extern "C" int st_host_alloc(size_t bytes, void **out) {
     void *d = NULL;
     if (hipHostGetDevicePointer(&d, *out, 0) == hipSuccess && d == *out) {
         std::lock_guard<std::mutex> lk(g_pin_mu);
-        g_pinned[(uintptr_t)*out] = bytes ? bytes : 1;
+        try {
+            g_pinned[(uintptr_t)*out] = bytes ? bytes : 1;
+        } catch (const std::bad_alloc &) {
+            (void)hipHostFree(*out);
+            *out = NULL;
+            return set_err(ST_ERR_MEMORY, "out of host memory");
+        }
     }
     return ST_OK;
 }

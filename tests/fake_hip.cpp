@@ -31,6 +31,13 @@ static std::mutex g_mu;
 static std::map<const void *, std::string> g_kernels;
 static std::map<uintptr_t, size_t> g_device, g_host;
 
+/* allocations of this file are not the library's */
+static thread_local int t_own;
+struct Own {
+    Own() { t_own++; }
+    ~Own() { t_own--; }
+};
+
 static hipError_t call(const char *name, void **args = nullptr) {
     if (g_hook) g_hook(name, args);
     if (g_fail_in > 0 && g_fail_name == name && --g_fail_in == 0) return 999;
@@ -39,6 +46,7 @@ static hipError_t call(const char *name, void **args = nullptr) {
 static hipError_t take(std::map<uintptr_t, size_t> &m, void **p, size_t n) {
     *p = calloc(1, n ? n : 1);
     if (!*p) return 2;
+    Own own;
     std::lock_guard<std::mutex> lk(g_mu);
     m[(uintptr_t)*p] = n;
     return 0;
@@ -58,7 +66,7 @@ static bool within(const std::map<uintptr_t, size_t> &m, const void *p) {
 
 /* the library's own allocations (it finds this operator before libstdc++'s) */
 void *operator new(size_t n) {
-    if (g_new_in > 0 && --g_new_in == 0) throw std::bad_alloc();
+    if (!t_own && g_new_in > 0 && --g_new_in == 0) throw std::bad_alloc();
     void *p = malloc(n ? n : 1);
     if (!p) throw std::bad_alloc();
     return p;
@@ -113,7 +121,12 @@ hipError_t __hipPopCallConfiguration(dim3_ *grid, dim3_ *block, size_t *lds, voi
     return 0;
 }
 hipError_t hipLaunchKernel(const void *f, dim3_, dim3_, void **args, size_t, void *) {
-    return call(("launch " + g_kernels[f]).c_str(), args);
+    std::string name;
+    {
+        Own own;
+        name = "launch " + g_kernels[f];
+    }
+    return call(name.c_str(), args);
 }
 
 hipError_t hipGetDeviceCount(int *n) {

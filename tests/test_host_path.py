@@ -35,6 +35,8 @@ class Fake:
             digits = "".join(c for c in name[9:12] if c.isdigit())
             name = "launch " + name[9 + len(digits):][:int(digits)]
         self.log.append(name)
+        if name == "launch k_mb_emit":   # the height that a device build reports
+            C.cast(C.cast(args[5], C.POINTER(C.c_void_p))[0], C.POINTER(C.c_uint32))[0] = 20
         if self.act:
             self.act(name, args)
 
@@ -175,6 +177,51 @@ def copying_threads_start_when_there_is_something_to_copy(fake, st):
     st.render(ds, view)
     assert seen[0][0] == before and seen[0][1] < 1.0, (before, seen[0])
     assert max(n for n, _ in seen) > before, seen   # the ring was used
+
+
+def _each_allocation(fake, st, call, at=None):
+    """call() once for each of the library's C++ allocations (from the first `at` on), that one failing: an error or a
+    result, and the process goes on. Returns how many there are."""
+    for nth in range(1, 400):
+        def act(name, args, nth=nth):
+            if name == at:
+                fake.so.fake_new_fail(nth)
+                fake.act = None
+        fake.act = act if at else None
+        if not at:
+            fake.so.fake_new_fail(nth)
+        try:
+            call()
+        except st.SlimTracinError:
+            pass
+        left = fake.so.fake_new_left()
+        fake.so.fake_new_fail(0)
+        if left > 0:
+            return nth - 1
+    raise AssertionError("no end of allocations")
+
+
+@case
+def running_out_of_host_memory_is_an_error(fake, st):
+    import numpy as np
+    from slimtracin_amd.scene import MODE_BEAUTY, MODE_DEPTH, make_view
+    ds = st.DeviceScene(st.gen_implicit(3))
+    view = make_view(width=1000, height=700, mode=MODE_DEPTH)
+    want = st.render(ds, view)
+    assert _each_allocation(fake, st, lambda: st.render(ds, view), at="launch k_deliver") >= 8
+    assert _each_allocation(fake, st, lambda: st.render(ds, view)) >= 15
+    got = st.render(ds, view)
+    assert got[0].tobytes() == want[0].tobytes()
+    scenes, views, outs = _mixed_batch(st)
+    st.render_batch_bgra8(scenes, views, outs=outs)
+    assert _each_allocation(fake, st, lambda: st.render_batch_bgra8(scenes, views, outs=outs)) >= 15
+    blob = st.gen_mesh_scene(3, 90000)
+    with_meshes = lambda: st.DeviceScene(blob, mesh_lbvh=True).close()   # noqa: E731
+    with_meshes()
+    bytes_before = fake.so.fake_device_bytes()
+    assert _each_allocation(fake, st, with_meshes) >= 8
+    assert fake.so.fake_device_bytes() == bytes_before
+    assert _each_allocation(fake, st, lambda: st.pinned_empty(100, np.uint8)) >= 1
 
 
 @pytest.fixture(scope="module")
