@@ -87,7 +87,8 @@ static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const
             e = download ? hipMemcpyAsync(s.host, s.dev, s.bytes, hipMemcpyDeviceToHost, stream)
                          : hipMemcpyAsync(s.dev, s.host, s.bytes, hipMemcpyHostToDevice, stream);
         }
-        return e != hipSuccess ? e : hipStreamSynchronize(stream);
+        const hipError_t w = hipStreamSynchronize(stream);
+        return e != hipSuccess ? e : w;
     };
     if (in_range) *in_range = true;
     if (in_order || total < COPY_MIN_BYTES || !copy_ring_ready(ring)) return plain();
@@ -175,8 +176,11 @@ static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const
                 if (e == hipSuccess) open[old + COPY_SLOTS].store(1, std::memory_order_release);
             }
         }
-        /* the ring is free again when the call returns */
-        if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    }
+    /* the ring is free again when the call returns, also with an error */
+    if (!download || e != hipSuccess) {
+        const hipError_t w = hipStreamSynchronize(stream);
+        if (e == hipSuccess) e = w;
     }
     stop = 1;
     for (std::thread &t : team) t.join();

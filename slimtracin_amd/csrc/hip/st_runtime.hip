@@ -2392,7 +2392,7 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
                 c->graph_exec = nullptr;
                 return set_err(ST_ERR_HIP, "graph instantiation failed: %s", hipGetErrorString(ie));
             }
-            c->graph_sig = sig;
+            c->graph_sig.swap(sig);
             g.graph_captures++;
         }
         if (timed) HIP_TRY(hipEventRecord(c->ev[0], c->stream));

@@ -224,6 +224,29 @@ def running_out_of_host_memory_is_an_error(fake, st):
     assert _each_allocation(fake, st, lambda: st.pinned_empty(100, np.uint8)) >= 1
 
 
+@case
+def a_failed_upload_has_waited_for_its_copies(fake, st):
+    """A copy or event of a large upload that fails: the copies before it are waited for before the scene's memory is
+    freed or the ring's slots are written again."""
+    blob = st.gen_mesh_scene(3, 200000)
+    for flags in (dict(mesh_binned=True), dict(mesh_lbvh=True)):
+        st.DeviceScene(blob, **flags).close()
+        for name in ("hipMemcpyAsync", "hipEventRecord", "hipEventSynchronize"):
+            for nth in (1, 2, 4, 7):
+                fake.so.fake_fail(name.encode(), nth)
+                del fake.log[:]
+                try:
+                    st.DeviceScene(blob, **flags).close()
+                    assert nth > 2, (flags, name)   # so few calls of this kind
+                    fake.so.fake_fail(b"", 0)
+                    break
+                except st.SlimTracinError:
+                    pass
+                last = max([i for i, c in enumerate(fake.log) if c == "hipMemcpyAsync"], default=-1)
+                after = fake.log[last + 1:]
+                assert after.index("hipStreamSynchronize") < after.index("hipFree"), (flags, name, nth, fake.log)
+
+
 @pytest.fixture(scope="module")
 def fake_so(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
