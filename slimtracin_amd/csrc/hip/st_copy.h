@@ -56,6 +56,7 @@ struct CopySpan {
     char *dev, *host;
     size_t bytes;
     uint32_t limit;   /* an upload of indices: each 32-bit word has to be below it (0: not indices) */
+    bool direct;      /* set by copy_spans: not pageable memory */
 };
 
 static inline bool words_below(const char *p, size_t bytes, uint32_t limit) {
@@ -65,33 +66,56 @@ static inline bool words_below(const char *p, size_t bytes, uint32_t limit) {
     return !over;
 }
 
-/* Copy the spans between pageable host memory and the device on `stream`,
-   after the work queued there; complete when the call returns. Plain copy
-   calls where the whole is small or the ring or its threads cannot be had,
-   and where the spans have to be copied one after another (in_order: they
-   overlap).
+/* Whether the runtime knows the memory (page-locked by whomever, or the
+   device's): a plain copy call then runs at the link's rate, with no bytes
+   for threads to move. */
+static inline bool copy_known(const char *p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
+/* Copy the spans between host memory and the device on `stream`, after the
+   work queued there; complete when the call returns. Plain copy calls for
+   memory that is not pageable, where the whole is small or the ring or its
+   threads cannot be had, and where the spans have to be copied one after
+   another (in_order: they overlap).
    *in_range (uploads) tells whether all indices are below their limits: the
    threads look while they have the bytes at hand (24 MB of indices by
    themselves, on one thread: 2 ms). */
-static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const CopySpan *spans, size_t nspans,
+static inline hipError_t copy_spans(hipStream_t stream, CopyRing *ring, CopySpan *spans, size_t nspans,
                                        bool download, bool in_order, bool *in_range = nullptr) {
     size_t total = 0;
     for (size_t k = 0; k < nspans; k++) total += spans[k].bytes;
     std::atomic<uint32_t> over(0);
-    auto plain = [&]() {
-        hipError_t e = hipSuccess;
-        for (size_t k = 0; k < nspans; k++) {
+    hipError_t e = hipSuccess;
+    auto copy_calls = [&](bool direct) {
+        for (size_t k = 0; k < nspans && e == hipSuccess; k++) {
             const CopySpan &s = spans[k];
-            if (!s.bytes || e != hipSuccess) continue;
+            if (!s.bytes || s.direct != direct) continue;
             if (in_range && s.limit && !words_below(s.host, s.bytes, s.limit)) *in_range = false;
             e = download ? hipMemcpyAsync(s.host, s.dev, s.bytes, hipMemcpyDeviceToHost, stream)
                          : hipMemcpyAsync(s.dev, s.host, s.bytes, hipMemcpyHostToDevice, stream);
         }
+    };
+    auto plain = [&]() {
+        copy_calls(false);
         const hipError_t w = hipStreamSynchronize(stream);
         return e != hipSuccess ? e : w;
     };
     if (in_range) *in_range = true;
-    if (in_order || total < COPY_MIN_BYTES || !copy_ring_ready(ring)) return plain();
+    for (size_t k = 0; k < nspans; k++) spans[k].direct = false;
+    if (in_order || total < COPY_MIN_BYTES) return plain();
+    for (size_t k = 0; k < nspans; k++) {
+        CopySpan &s = spans[k];
+        s.direct = s.bytes && !s.limit && copy_known(s.host) && copy_known(s.host + s.bytes - 1);
+        if (s.direct) total -= s.bytes;
+    }
+    copy_calls(true);
+    if (e != hipSuccess || total < COPY_MIN_BYTES || !copy_ring_ready(ring)) return plain();
     std::vector<CopySpan> chunk;
     /* A chunk's state: `open` says that its slot may be moved by a thread (the
        download into it is done, or the upload before it has left it), `moved`
@@ -101,9 +125,9 @@ static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const
     try {
         chunk.reserve(total / COPY_SLOT_BYTES + nspans);
         for (size_t k = 0; k < nspans; k++)
-            for (size_t at = 0; at < spans[k].bytes; at += COPY_SLOT_BYTES)
+            for (size_t at = 0; at < spans[k].bytes && !spans[k].direct; at += COPY_SLOT_BYTES)
                 chunk.push_back({spans[k].dev + at, spans[k].host + at,
-                                 std::min(spans[k].bytes - at, (size_t)COPY_SLOT_BYTES), spans[k].limit});
+                                 std::min(spans[k].bytes - at, (size_t)COPY_SLOT_BYTES), spans[k].limit, false});
         std::vector<std::atomic<uint32_t>>(chunk.size()).swap(open);
         std::vector<std::atomic<uint32_t>>(chunk.size()).swap(moved);
         team.reserve(COPY_THREADS);
@@ -135,7 +159,6 @@ static inline hipError_t copy_pageable(hipStream_t stream, CopyRing *ring, const
         }
         return !team.empty();
     };
-    hipError_t e = hipSuccess;
     auto wait_moved = [&](uint32_t i) {
         while (!moved[i].load(std::memory_order_acquire)) std::this_thread::yield();
     };

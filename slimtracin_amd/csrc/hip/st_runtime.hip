@@ -1578,7 +1578,7 @@ static int build_device_meshes(StSceneHandle *h) {
         size_t nspans = 0;
         for (int k = 0; k < 6; k++) {
             if (!up[k].src || !up[k].bytes) continue;
-            spans[nspans++] = {p, (char *)up[k].src, up[k].bytes, up[k].limit};
+            spans[nspans++] = {p, (char *)up[k].src, up[k].bytes, up[k].limit, false};
             *up[k].dst = p;
             p += round256(up[k].bytes);
         }
@@ -1587,7 +1587,7 @@ static int build_device_meshes(StSceneHandle *h) {
             rc = set_err(ST_ERR_SCENE, "invalid scene: mesh index out of range");
             break;
         }
-        if (copy_pageable(g.main.stream, &g.main.ring, spans, nspans, false, false, &in_range) != hipSuccess) {
+        if (copy_spans(g.main.stream, &g.main.ring, spans, nspans, false, false, &in_range) != hipSuccess) {
             rc = set_err(ST_ERR_HIP, "mesh geometry upload failed");
             break;
         }
@@ -1710,8 +1710,8 @@ extern "C" int st_scene_upload(StSceneHandle *h) {
     CopySpan spans[sizeof parts / sizeof parts[0]];
     size_t nspans = 0;
     for (size_t i = 0; i < sizeof parts / sizeof parts[0]; i++)
-        if (parts[i].bytes) spans[nspans++] = {b + parts[i].off, (char *)parts[i].src, parts[i].bytes, 0};
-    HIP_TRY(copy_pageable(g.main.stream, &g.main.ring, spans, nspans, false, false));
+        if (parts[i].bytes) spans[nspans++] = {b + parts[i].off, (char *)parts[i].src, parts[i].bytes, 0, false};
+    HIP_TRY(copy_spans(g.main.stream, &g.main.ring, spans, nspans, false, false));
     if (sc->mesh_count) {
         float *ma = (float *)malloc(24ull * sc->mesh_count);
         for (uint32_t m = 0; m < sc->mesh_count; m++) {
@@ -2418,14 +2418,14 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
     for (uint32_t i = 0; i < n; i++) {
         size_t px = (size_t)hv[i].dv.width1 * hv[i].dv.height1;
         if (pixels_host && pixels_host[i] && !own_px[i])
-            spans.push_back({(char *)reqs_h[i].v.pixels, (char *)pixels_host[i], px * 24, 0});
+            spans.push_back({(char *)reqs_h[i].v.pixels, (char *)pixels_host[i], px * 24, 0, false});
         if (hits_host && hits_host[i] && want_hits && !own_hits[i])
-            spans.push_back({(char *)reqs_h[i].v.hits, (char *)hits_host[i], px * 16, 0});
+            spans.push_back({(char *)reqs_h[i].v.hits, (char *)hits_host[i], px * 16, 0, false});
         if (reqs_h[i].bgra && !own_bgra[i])
             spans.push_back({(char *)reqs_h[i].bgra, (char *)bgra_host[i],
-                             (size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4, 0});
+                             (size_t)(hv[i].dv.width1 - 1) * (hv[i].dv.height1 - 1) * 4, 0, false});
     }
-    if (!spans.empty()) HIP_TRY(copy_pageable(c->stream, &c->ring, spans.data(), spans.size(), true, !apart));
+    if (!spans.empty()) HIP_TRY(copy_spans(c->stream, &c->ring, spans.data(), spans.size(), true, !apart));
     HIP_TRY(hipStreamSynchronize(c->stream));
     guard.pending = false;
     c->last_redo = (uint32_t)cnt_h[3 * (size_t)n + 1];

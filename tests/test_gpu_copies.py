@@ -10,6 +10,7 @@ import struct
 
 import numpy as np
 import pytest
+import torch
 
 import slimtracin_amd as st
 from slimtracin_amd.scene import MODE_DEPTH, PIXEL_DTYPE, blob_mesh_info, make_view
@@ -56,3 +57,22 @@ def test_indices_out_of_range_are_refused(tris, which, place):
         st.DeviceScene(bytes(blob), mesh_lbvh=True)
     struct.pack_into("<I", blob, at, limit - 1)
     st.DeviceScene(bytes(blob), mesh_lbvh=True).close()
+
+
+@pytest.mark.parametrize("whose", ["another library's", "unaligned"])
+@pytest.mark.parametrize("w,h", [(599, 291), (1439, 1079)])
+def test_downloads_into_page_locked_memory_that_the_device_does_not_write(scene, whose, w, h):
+    """Copied directly, next to hit records in pageable memory that take the ring."""
+    view = make_view(width=w, height=h, mode=MODE_DEPTH, position=(0.0, 7.0, -11.0), pitch=-0.2)
+    n = (w + 1) * (h + 1)
+    want, want_hits, _ = st.render(scene, view)
+    if whose == "unaligned":
+        block = st.pinned_empty(24 * n + 4, np.uint8)
+    else:
+        block = torch.zeros(24 * n + 4, dtype=torch.uint8, pin_memory=True).numpy()
+    for at in (0, 4) if whose != "unaligned" else (4,):
+        block[:] = 0x5A
+        out = block[at:at + 24 * n].view(PIXEL_DTYPE)
+        _, hits, _ = st.render(scene, view, out=out)
+        assert out.tobytes() == want.tobytes() and hits.tobytes() == want_hits.tobytes()
+        assert (block[:at] == 0x5A).all() and (block[at + 24 * n:] == 0x5A).all()

@@ -247,6 +247,40 @@ def a_failed_upload_has_waited_for_its_copies(fake, st):
     assert failed > 12, failed
 
 
+@case
+def page_locked_memory_of_others_is_copied_directly(fake, st):
+    """Outputs that the device does not write itself but that a copy call can reach at the link's rate: one call each,
+    with no threads; pageable ones of the same call still take the ring."""
+    import numpy as np
+    from slimtracin_amd.scene import HIT_DTYPE, MODE_DEPTH, PIXEL_DTYPE, make_view
+    ds = st.DeviceScene(st.gen_implicit(3))
+    w, h = 999, 699
+    n = (w + 1) * (h + 1)
+    view = make_view(width=w, height=h, mode=MODE_DEPTH)
+    before, copies, threads = _threads(), [], []
+
+    def act(name, args):
+        if name == "hipMemcpyAsync":
+            copies.append((args[0], args[2]))
+        if name in ("hipEventSynchronize", "hipStreamSynchronize"):
+            threads.append(_threads())
+
+    foreign = fake.so.fake_host_alloc(C.c_size_t(24 * n))
+    unaligned = st.pinned_empty(24 * n + 4, np.uint8)[4:]
+    hits = np.empty(n, HIT_DTYPE)
+    st.render(ds, view)
+    fake.act = act
+    for out in (foreign, unaligned.ctypes.data):
+        for hp in (None, hits.ctypes.data):
+            del copies[:], threads[:]
+            assert st.lib().st_render(ds.handle, C.c_void_p(view.ctypes.data), C.c_void_p(out), C.c_void_p(hp), None) == 0
+            assert (out, 24 * n) in copies, copies
+            if hp:
+                assert len(copies) > 4 and max(threads) > before
+            else:
+                assert len(copies) == 1 and max(threads) == before
+
+
 @pytest.fixture(scope="module")
 def fake_so(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
