@@ -5,8 +5,8 @@
  * runtime with one thread moving the bytes: 52 MB of mesh geometry took 3.8
  * ms (14 GB/s on a link of 57), 15 MB of fresh pages for hit records 1.1 ms,
  * most of it page faults. Here the bytes go through a ring of page-locked
- * slots with several threads at its host side: 1.2 and 0.5 ms. Copies under
- * COPY_MIN_BYTES keep the call, which then costs less than the threads.
+ * slots with several threads at its host side: 1.2 and 0.5 ms. Smaller copies
+ * keep the call, which then costs less than the threads.
  */
 #ifndef ST_COPY_H
 #define ST_COPY_H
@@ -24,7 +24,13 @@
 
 #define COPY_SLOTS 8u
 #define COPY_SLOT_BYTES (2u << 20)
-#define COPY_MIN_BYTES (4u << 20)
+/* Bytes from which the ring is the quicker. A depth frame into pageable
+   memory, ring and call: 2 MiB 216 and 178 us, 3 MiB 269 and 257, 4 MiB 314
+   and 328, 8 MiB 460 and 605. Creating a scene with a device-built mesh (its
+   geometry checked by the threads, or on one): 11.9 MB 1010 and 922 us, 15.9
+   MB 1155 and 1070, 31.8 MB 2075 and 2300, 49.6 MB 2765 and 3515. */
+#define COPY_MIN_DOWNLOAD (4u << 20)
+#define COPY_MIN_UPLOAD (24u << 20)
 #define COPY_THREADS 8u
 
 /* A launch context's ring: 16 MiB of page-locked memory and an event per
@@ -88,6 +94,7 @@ static inline bool copy_known(const char *p) {
    themselves, on one thread: 2 ms). */
 static inline hipError_t copy_spans(hipStream_t stream, CopyRing *ring, CopySpan *spans, size_t nspans,
                                        bool download, bool in_order, bool *in_range = nullptr) {
+    const size_t least = download ? COPY_MIN_DOWNLOAD : COPY_MIN_UPLOAD;
     size_t total = 0;
     for (size_t k = 0; k < nspans; k++) total += spans[k].bytes;
     std::atomic<uint32_t> over(0);
@@ -108,14 +115,14 @@ static inline hipError_t copy_spans(hipStream_t stream, CopyRing *ring, CopySpan
     };
     if (in_range) *in_range = true;
     for (size_t k = 0; k < nspans; k++) spans[k].direct = false;
-    if (in_order || total < COPY_MIN_BYTES) return plain();
+    if (in_order || total < least) return plain();
     for (size_t k = 0; k < nspans; k++) {
         CopySpan &s = spans[k];
         s.direct = s.bytes && !s.limit && copy_known(s.host) && copy_known(s.host + s.bytes - 1);
         if (s.direct) total -= s.bytes;
     }
     copy_calls(true);
-    if (e != hipSuccess || total < COPY_MIN_BYTES || !copy_ring_ready(ring)) return plain();
+    if (e != hipSuccess || total < least || !copy_ring_ready(ring)) return plain();
     std::vector<CopySpan> chunk;
     /* A chunk's state: `open` says that its slot may be moved by a thread (the
        download into it is done, or the upload before it has left it), `moved`

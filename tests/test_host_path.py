@@ -215,7 +215,7 @@ def running_out_of_host_memory_is_an_error(fake, st):
     scenes, views, outs = _mixed_batch(st)
     st.render_batch_bgra8(scenes, views, outs=outs)
     assert _each_allocation(fake, st, lambda: st.render_batch_bgra8(scenes, views, outs=outs)) >= 15
-    blob = st.gen_mesh_scene(3, 90000)
+    blob = st.gen_mesh_scene(3, 600000)
     with_meshes = lambda: st.DeviceScene(blob, mesh_lbvh=True).close()   # noqa: E731
     with_meshes()
     bytes_before = fake.so.fake_device_bytes()
@@ -228,7 +228,7 @@ def running_out_of_host_memory_is_an_error(fake, st):
 def a_failed_upload_has_waited_for_its_copies(fake, st):
     """A copy or event of a large upload that fails: the copies before it are waited for before the scene's memory is
     freed or the ring's slots are written again."""
-    blob, failed = st.gen_mesh_scene(3, 200000), 0
+    blob, failed = st.gen_mesh_scene(3, 600000), 0
     for flags in (dict(mesh_binned=True), dict(mesh_lbvh=True)):
         st.DeviceScene(blob, **flags).close()
         for name in ("hipMemcpyAsync", "hipEventRecord", "hipEventSynchronize"):
@@ -279,6 +279,25 @@ def page_locked_memory_of_others_is_copied_directly(fake, st):
                 assert len(copies) > 4 and max(threads) > before
             else:
                 assert len(copies) == 1 and max(threads) == before
+
+
+@case
+def only_large_copies_take_threads(fake, st):
+    """Uploads below 24 MiB and downloads below 4 MiB are plain calls, on the calling thread."""
+    from slimtracin_amd.scene import MODE_DEPTH, make_view
+    threads = []
+    fake.act = lambda name, args: threads.append(_threads())
+    before = _threads()
+    for triangles, ring in ((400000, False), (600000, True)):
+        blob = st.gen_mesh_scene(3, triangles)
+        del threads[:]
+        st.DeviceScene(blob, mesh_lbvh=True).close()
+        assert (max(threads) > before) == ring, (triangles, before, max(threads))
+    ds = st.DeviceScene(st.gen_implicit(3))
+    for width, ring in ((417, False), (418, True)):
+        del threads[:]
+        st.render(ds, make_view(width=width, height=417, mode=MODE_DEPTH), hits=False)
+        assert (max(threads) > before) == ring, (width, before, max(threads))
 
 
 @pytest.fixture(scope="module")
