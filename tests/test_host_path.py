@@ -300,6 +300,25 @@ def only_large_copies_take_threads(fake, st):
         assert (max(threads) > before) == ring, (width, before, max(threads))
 
 
+@case
+def a_mesh_build_keeps_no_device_memory(fake, st):
+    """What a device build needs besides the scene is given back before the scene's creation returns."""
+    from slimtracin_amd.server import Server
+    for triangles in (500, 100000, 600000):
+        blob = st.gen_mesh_scene(3, triangles)
+        before = fake.so.fake_device_bytes()
+        ds = st.DeviceScene(blob, mesh_lbvh=True)
+        assert fake.so.fake_device_bytes() - before == ds.info().device_bytes
+        ds.close()
+        assert fake.so.fake_device_bytes() == before
+        srv = Server()
+        with_server = fake.so.fake_device_bytes()
+        srv.remove_scene(srv.add_scene(blob, mesh_lbvh=True))
+        assert fake.so.fake_device_bytes() == with_server
+        srv.close()
+        assert fake.so.fake_device_bytes() == before
+
+
 @pytest.fixture(scope="module")
 def fake_so(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
