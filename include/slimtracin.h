@@ -213,8 +213,8 @@ void st_host_free(void *p);
 int st_resolve_bgra8(const StFloatPixel *grid, uint32_t grid_w, uint32_t grid_h, uint32_t *out);
 
 /* As st_render_batch without downloads; returns the duration of the
-   launch's device work (all stages) measured with HIP events on the launch
-   stream. */
+   launch's device work (the upload, preparation and all stages) measured with
+   HIP events on the launch stream. */
 int st_render_timed(StSceneHandle *const *scenes, const StView *views, uint32_t n, uint32_t flags, float *kernel_ms,
                     StRayCounts *counts);
 

@@ -2259,16 +2259,16 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
         return hipEventRecord(c->stage_ev[marks++], c->stream);
     };
     /* everything from the upload to the ray counts; the same stream work is
-       what a graph captures. ev[0] .. ev[1] brackets every kernel of the
-       launch (the render time st_render_timed reports). */
+       what a graph captures. ev[0] .. ev[1] brackets all of it, the upload
+       too (the render time st_render_timed reports). */
     auto enqueue = [&]() -> int {
+        if (!graph && timed) HIP_TRY(hipEventRecord(c->ev[0], c->stream));
         hipLaunchKernelGGL(k_setup, dim3(setup_blocks(up)), dim3(SETUP_THREADS), 0, c->stream,
                            (const uint4 *)c->staging_dev, (uint4 *)blk, (uint32_t)(up / 16), cnt_d, 3 * n + 2,
                            c->tile_counter, CLAIM_WORDS, w.ctr, (uint32_t *)(c->cost_sum + 1));
         static_assert(BOUNCE_CLAIM < ORDER_CLAIM && ORDER_CLAIM + 1 < XCD_CLAIM &&
                           XCD_CLAIM + 8 * XCD_CLAIM_STRIDE <= CLAIM_WORDS,
                       "claim counters share the zeroed words");
-        if (!graph && timed) HIP_TRY(hipEventRecord(c->ev[0], c->stream));
         if (use_history) {
             hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, c->cost_sum, 1u);
             hipLaunchKernelGGL(k_cost_total, dim3(cost_blocks), dim3(COST_THREADS), 0, c->stream,

@@ -319,6 +319,23 @@ def a_mesh_build_keeps_no_device_memory(fake, st):
         assert fake.so.fake_device_bytes() == before
 
 
+@case
+def a_timed_launch_is_timed_from_its_upload_on(fake, st):
+    """Launched kernel by kernel or as a graph, the time covers the same work."""
+    from slimtracin_amd.scene import MODE_BEAUTY, make_view
+    ds = st.DeviceScene(st.gen_pbr(3, 10))
+    view = make_view(width=90, height=70, mode=MODE_BEAUTY, depth=3)
+    for stages in (False, True):
+        for graph in (False, True):
+            for _ in range(2):
+                del fake.log[:]
+                st.render_timed([ds], view, stages=stages, graph=graph)
+                work = [i for i, c in enumerate(fake.log) if c == "hipGraphLaunch" or
+                        (c.startswith("launch ") and c != "launch k_deliver" and not graph)]
+                marks = [i for i, c in enumerate(fake.log) if c == "hipEventRecord"]
+                assert marks[0] < work[0] and work[-1] < marks[-1], (stages, graph, fake.log)
+
+
 @pytest.fixture(scope="module")
 def fake_so(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
