@@ -904,17 +904,27 @@ __device__ static inline __attribute__((always_inline)) void drain_queue(const K
    64. The lanes of a chunk go different ways and wait for each other, at
    every primitive and on every level of a tree, so a short queue ends sooner
    spread over idle waves; but each of those fetches code, primitives and
-   nodes anew. Stage times with chunks of at least 64, 16 and 4:
-     25 instances, 320x200: 0.71, 0.53, 0.43 ms; 64 instances, 1280x720
-       (9,400 pixels): 2.10, 1.67, 1.58 (of at least 1: 1.61)
-     one mesh of 450,000 triangles, 320x200: 0.66, 0.57, 0.62; 72,000: 0.55,
-       0.46, 0.50; 18,000, 1000x500: 0.42, 0.39, 0.37
-     one mesh of 320 triangles, 320x200: 0.23, 0.23, 0.31; 160x120: 0.24,
-       0.27, 0.28; 4,500, 160x120: 0.34, 0.36, 0.37
-   hence bounce_width: 4 with several primitives, otherwise 16 for large
-   meshes and 64 for small ones; a launch takes the least of its scenes'. */
+   nodes anew. Stage times in ms with chunks of at least 64, 16 and 4, at
+   160x120 and 1280x720:
+     4 mesh primitives of 6: 0.88 0.73 0.56, 0.72 0.61 0.63 (meshes of 1,000
+       triangles); of 5: 0.51 0.45 0.34, 0.63 0.52 0.46; 24 of 25: 0.70 0.53
+       0.38, 0.62 0.56 0.54; 64 instances, 1280x720: 2.10 1.67 1.58
+     one of 6: 0.047 0.045 0.054, 0.051 0.058 0.075 (1,000 triangles); 0.13
+       0.14 0.17, 0.17 0.17 0.17 (320); of 16: 0.21 0.24 0.23, 0.24 0.24 0.27
+     one of 6, 320x200: 450,000 triangles 0.66 0.57 0.62; 72,000 0.55 0.46
+       0.50; 18,000 at 160x120 0.16 0.17 0.20, 1000x500 0.42 0.39 0.37
+     none of 8: 0.039 0.040 0.056, 0.041 0.049 0.063; of 16: 0.22 0.21 0.17,
+       0.20 0.20 0.25 and 0.13 0.13 0.15, 0.12 0.11 0.12; of 24: 0.28 0.24
+       0.20, 0.25 0.25 0.26; of 32: 0.32 0.27 0.23, 0.29 0.27 0.27; of 300:
+       1.23 0.82 0.64, 0.91 0.70 0.71
+   hence bounce_width: 4 with several mesh primitives (each a traversal of its
+   own) or very many primitives, 16 in between and for large meshes, 64
+   otherwise. A launch takes the least of its scenes': one of 320 triangles
+   with one of 24 instances, 160x120 each, 0.64 0.53 0.37, with a small frame
+   of 16 implicit primitives 0.13 0.14 0.18. */
 static uint32_t bounce_width(const StScene *sc) {
-    return sc->prim_count >= 8u ? 4u : sc->tri_total >= 16384u ? 16u : 64u;
+    if (sc->mesh_prims >= 4u || sc->prim_count >= 32u) return 4u;
+    return sc->prim_count >= 16u || sc->tri_total >= 16384u ? 16u : 64u;
 }
 __global__ void __launch_bounds__(BLOCK_THREADS) K_BOUNCE_ATTR k_bounce(const StDScene *__restrict__ scenes,
                                                           const KReq *__restrict__ reqs, uint32_t nreq, KWave w,
@@ -1812,11 +1822,7 @@ extern "C" int st_scene_set_prims(StSceneHandle *h, const StPrimRec *recs, uint3
             return set_err(ST_ERR_ARG, "primitive %u: mesh_id out of range", first + i);
     }
     for (uint32_t i = 0; i < count; i++) sc->prims[first + i] = st_prim_from_rec(recs + i);
-    sc->has_emissive_quads = 0;
-    for (uint32_t i = 0; i < sc->prim_count; i++) {
-        uint32_t mid = (sc->prims[i].flags_mat >> 8) & 0xFFu;
-        if (sc->prims[i].type == ST_PRIM_QUAD && (sc->mats[mid].bits & ST_EMISSIVE)) sc->has_emissive_quads = 1;
-    }
+    st_scene_kinds(sc);
     h->dev.has_emissive_quads = sc->has_emissive_quads;
     HIP_TRY(hipMemcpyAsync((void *)(h->dev.prims + first), sc->prims + first, count * sizeof(StDPrim),
                            hipMemcpyHostToDevice, g.main.stream));

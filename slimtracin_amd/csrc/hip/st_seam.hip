@@ -263,11 +263,7 @@ static int seam_build(StSceneHandle *h) {
 
 static void refresh_emissive(StSceneHandle *h) {
     StScene *sc = h->host;
-    sc->has_emissive_quads = 0;
-    for (uint32_t i = 0; i < sc->prim_count; i++) {
-        uint32_t mid = (sc->prims[i].flags_mat >> 8) & 0xFFu;
-        if (sc->prims[i].type == ST_PRIM_QUAD && (sc->mats[mid].bits & ST_EMISSIVE)) sc->has_emissive_quads = 1;
-    }
+    st_scene_kinds(sc);
     h->dev.has_emissive_quads = sc->has_emissive_quads;
 }
 

@@ -50,7 +50,7 @@ typedef struct StScene {
     uint32_t mip_total;
     uint8_t *texels;
     uint64_t texel_bytes;
-    uint32_t has_emissive_quads;
+    uint32_t has_emissive_quads, mesh_prims;   /* over the primitives as they are now (st_scene_kinds) */
     uint32_t mesh_stack_size;
     uint32_t scene_real_height;    /* levels of the scene BVH as walked */
     /* meshes whose BVH and triangle records are built on the device: their
@@ -107,6 +107,10 @@ typedef struct StSceneParts {
 #define ST_MESH_BUILD_BINNED 2u
 /* ST_MESH_BUILD_DEVICE with the caller checking the meshes' indices */
 #define ST_MESH_BUILD_DEVICE_UNCHECKED 3u
+
+/* What launches want to know about all of the primitives; again whenever
+   primitives or materials change. */
+void st_scene_kinds(StScene *sc);
 
 /* Validate the parts and build the device-ready scene. Returns NULL on
    malformed input; *err (if given) receives a short reason. */

@@ -151,6 +151,15 @@ StDMat st_mat_from_rec(const StMaterialRec *q) {
 
 #define FAIL(msg) do { *err = (msg); st_scene_free(sc); return NULL; } while (0)
 
+void st_scene_kinds(StScene *sc) {
+    sc->has_emissive_quads = sc->mesh_prims = 0;
+    for (uint32_t i = 0; i < sc->prim_count; i++) {
+        uint32_t mid = (sc->prims[i].flags_mat >> 8) & 0xFFu;
+        if (sc->prims[i].type == ST_PRIM_QUAD && (sc->mats[mid].bits & ST_EMISSIVE)) sc->has_emissive_quads = 1;
+        sc->mesh_prims += sc->prims[i].type == ST_PRIM_MESH;
+    }
+}
+
 StScene *st_scene_from_parts(const StSceneParts *pp, const char **err) {
     const char *dummy;
     if (!err) err = &dummy;
@@ -343,10 +352,7 @@ StScene *st_scene_from_parts(const StSceneParts *pp, const char **err) {
         sc->scene_real_height = (uint32_t)real_height;
         if (real_height + 1 > ST_SCENE_STACK_MAX) FAIL("scene BVH deeper than the device traversal stack");
     }
-    for (uint32_t i = 0; i < P; i++) {
-        uint32_t mid = (sc->prims[i].flags_mat >> 8) & 0xFFu;
-        if (sc->prims[i].type == ST_PRIM_QUAD && (sc->mats[mid].bits & ST_EMISSIVE)) sc->has_emissive_quads = 1;
-    }
+    st_scene_kinds(sc);
     return sc;
 }
 

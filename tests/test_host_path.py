@@ -37,6 +37,8 @@ class Fake:
         self.log.append(name)
         if name == "launch k_mb_emit":   # the height that a device build reports
             C.cast(C.cast(args[5], C.POINTER(C.c_void_p))[0], C.POINTER(C.c_uint32))[0] = 20
+        if name == "launch k_deliver":   # the launch's ray counts and fault word
+            C.memset(C.cast(args[4], C.POINTER(C.c_void_p))[0], 0, 8 * self.u32(args, 5))
         if self.act:
             self.act(name, args)
 
@@ -336,6 +338,46 @@ def a_timed_launch_is_timed_from_its_upload_on(fake, st):
                 assert marks[0] < work[0] and work[-1] < marks[-1], (stages, graph, fake.log)
 
 
+@case
+def bounce_chunks_by_what_the_scenes_hold(fake, st):
+    """The least width of a launch's chunks, by its Beauty requests' scenes as their primitives are now."""
+    import numpy as np
+    import scenes as examples
+    from slimtracin_amd.scene import (MODE_BEAUTY, MODE_DEPTH, PRIM_BOX, PRIM_MESH, blob_prims, blob_with_prims,
+                                      make_view)
+
+    def crowd(n, meshes):
+        blob = examples.crowd(5, n)[0].to_blob()
+        prims = blob_prims(blob)
+        prims["type"] = PRIM_BOX
+        prims["type"][:meshes] = PRIM_MESH
+        return blob_with_prims(blob, prims)
+
+    widths = []
+    fake.act = lambda name, args: widths.append(fake.u32(args, 8)) if name == "launch k_bounce" else None
+    view = make_view(width=33, height=21, mode=MODE_BEAUTY, depth=3)
+    made = {}
+    for what, blob, want in [("8", crowd(8, 0), 64), ("15", crowd(15, 3), 64), ("16", crowd(16, 0), 16),
+                             ("31", crowd(31, 3), 16), ("32", crowd(32, 0), 4), ("4 meshes", crowd(5, 4), 4),
+                             ("320", st.gen_pbr(3, 4), 64), ("18000", st.gen_pbr(3, 30), 16)]:
+        ds = made[what] = st.DeviceScene(blob, mesh_binned=True)
+        for call in (st.render, st.render_noalloc):
+            del widths[:]
+            call(ds, view)
+            assert widths == [want], (what, widths)
+    for names, modes, want in [(("8", "320"), "bb", 64), (("8", "16", "18000"), "bbb", 16), (("8", "32", "320"), "bbb", 4),
+                               (("8", "32", "320"), "bdb", 64)]:
+        del widths[:]
+        st.render_batch([made[n] for n in names], np.concatenate(
+            [make_view(width=33, height=21, mode=MODE_BEAUTY if m == "b" else MODE_DEPTH, depth=3) for m in modes]))
+        assert widths == [want], (names, widths)
+    prims = blob_prims(crowd(5, 3))
+    made["4 meshes"].set_prims(np.ascontiguousarray(prims))
+    del widths[:]
+    st.render(made["4 meshes"], view)
+    assert widths == [64], widths
+
+
 @pytest.fixture(scope="module")
 def fake_so(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
@@ -352,7 +394,7 @@ def test_host_path(fake_so, name):
 
 
 if __name__ == "__main__":
-    sys.path.insert(0, os.path.dirname(HERE))
+    sys.path[:0] = [os.path.dirname(HERE), HERE]
     runtime = Fake(sys.argv[1])
     import slimtracin_amd as library
     library.init(0)
