@@ -538,12 +538,32 @@ __device__ static inline void resolve_share(const KReq *reqs, uint32_t nreq, uin
    13.7. */
 #define EARLY_BLOCKS 64u
 #define EARLY_CLAIMS 512u              /* the second kernel's counters, after the first's */
-/* Plain outputs and other requests' pixels below which one kernel is the
-   quicker: the drain between the two costs about 0.2 ms. 20 MB (20 requests):
-   2.97 ms in one kernel, 3.17 in two; 45 MB (160 of up to 700 pixels a side):
-   5.78, 5.76. */
+/* When it pays. Images of 48 MiB: the drain between the kernels costs about
+   0.2 ms (20 MB, 20 requests: 2.97 ms in one kernel, 3.17 in two; 45 MB, 160
+   of up to 700 pixels a side: 5.78, 5.76). And enough to render meanwhile,
+   since EARLY_BLOCKS blocks alone write at about half the link's rate:
+   early_bytes per pixel with a bounce stage. 58 MB and 166 MB of normals
+   images over 200,000 triangles, in one kernel and in two, in ms, at 16, 20,
+   24 and 32 bytes per such pixel (depth 2):
+     one mesh of 200,000 triangles   5.2 4.5, 4.7 4.0, 4.4 3.8, 4.0 3.7
+                                     13.9 11.6, 12.6 10.4, 11.6 9.9, 10.4 9.6
+     24 instances of 7,000 to 72,000 4.8 4.3, 4.5 4.2, 4.3 4.2, (28:) 4.1 4.1
+                                     12.4 11.1, 11.5 10.7, 10.7 10.3, 10.2 10.2
+     one mesh of 8,000               4.6 4.0, 4.2 3.8, 3.9 3.8, 3.5 3.6
+                                     12.4 10.8, 11.4 10.3, 10.5 9.9, 9.6 9.6
+     24 instances of 500 to 5,000    4.2 4.0, 3.9 3.9, 3.7 3.9, 3.4 3.8
+                                     11.1 10.5, 10.3 10.2, 9.7 9.9, 9.0 9.7
+     one mesh of 320                 4.1 3.9, 3.8 3.8, 3.6 3.7, (28:) 3.4 3.7
+                                     11.6 10.9, 10.7 10.5, 9.9 10.0, 9.5 9.8
+     implicit primitives             3.1 3.9, 3.0 3.8, 2.8 3.7, 2.7 3.6
+                                     8.2 9.6, 8.0 9.4, 7.7 9.8, 7.5 9.5
+   (implicit ones at 8: 3.6 4.5; 9.9 10.5.) Scenes whose meshes cover little
+   of the frame cannot be told from here (4 instances of 500 to 5,000, at 16:
+   3.9 4.2; 9.9 10.3). */
 #define EARLY_MIN_BYTES (48ull << 20)
-#define EARLY_MIN_PIXELS (1u << 21)
+static uint32_t early_bytes(const StScene *sc) {
+    return !sc->mesh_prims ? 0u : sc->tri_total >= 16384u ? 32u : 20u;
+}
 struct KEarly {
     uint32_t nreq;      /* the plain requests: the first of the launch's */
     uint32_t shares;    /* their resolve blocks; 0: nothing to deliver */
@@ -2446,7 +2466,7 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
 }
 
 /* A launch of plain requests (no bounce stage) with enough to deliver and of
-   others with enough to render meanwhile (EARLY_MIN_BYTES) runs in an order
+   others with enough to render meanwhile (early_bytes) runs in an order
    of its own, the plain ones first (KEarly); any other in the caller's. A
    captured graph keeps its outputs out of the graph, so its launches are not
    split; neither are those with an order of tiles of their own
@@ -2464,18 +2484,18 @@ static int launch_split(LaunchCtx *c, StSceneHandle *const *scenes, StHostView *
     };
     if (n < 2 || !apart || !persistent || c->graph_mode || sw.tune.cost_order == 1u) return straight();
     auto shaded = [&](uint32_t i) { return hv[i].dv.mode == ST_MODE_BEAUTY && hv[i].dv.depth > 1; };
-    uint64_t out = 0, px_shaded = 0;
+    uint64_t out = 0, covered = 0;
     for (uint32_t i = 0; i < n; i++) {
         const uint64_t w1 = hv[i].dv.width1, h1 = hv[i].dv.height1, px = w1 * h1;
         if (!scenes[i] || !scenes[i]->host || !scenes[i]->dbuf || w1 < 2 || h1 < 2) return straight();
         if (shaded(i)) {
-            px_shaded += px;
+            covered += px * early_bytes(scenes[i]->host);
             continue;
         }
         if (bgra_host && bgra_host[i] && deliverable(bgra_host[i], (w1 - 1) * (h1 - 1) * 4, IMAGE_ALIGN))
             out += (w1 - 1) * (h1 - 1) * 4;
     }
-    if (out < EARLY_MIN_BYTES || px_shaded < EARLY_MIN_PIXELS) return straight();
+    if (out < EARLY_MIN_BYTES || out > covered) return straight();
     std::vector<uint32_t> at(n);   /* launch order -> the caller's */
     uint32_t plain = 0, k = 0;
     for (uint32_t i = 0; i < n; i++)

@@ -103,8 +103,8 @@ def test_plain_requests_of_a_mixed_launch(call, abandon):
     sizes = [(1201, 701), (1, 1), (1600, 900), (640, 363), (1601, 900), (17, 5), (1024, 640)]
     modes = [MODE_BEAUTY, MODE_NORMALS, MODE_NORMALS, MODE_DEPTH, MODE_BEAUTY, MODE_BEAUTY, MODE_UVS]
     if call == "windows":   # enough bytes that the images go out early; grids and hit records always do
-        sizes += [(3201, 2003), (3199, 1999)]
-        modes += [MODE_UVS, MODE_NORMALS]
+        sizes += [(3201, 2003), (3199, 1999), (1601, 1001)]   # (and enough pixels with a bounce stage to do so)
+        modes += [MODE_UVS, MODE_NORMALS, MODE_BEAUTY]
     grid = [(w + 1) * (h + 1) for w, h in sizes]
     views = np.concatenate([make_view(width=w, height=h, mode=m, depth=0 if w == 17 else 2,
                                      position=(0.0, 3.0, -9.0), pitch=-0.1) for (w, h), m in zip(sizes, modes)])

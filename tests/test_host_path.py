@@ -378,6 +378,40 @@ def bounce_chunks_by_what_the_scenes_hold(fake, st):
     assert widths == [64], widths
 
 
+@case
+def launches_are_split_when_there_is_enough_to_render_meanwhile(fake, st):
+    """By the bytes of the plain requests' images and the pixels, and scenes, of the others."""
+    import numpy as np
+    from slimtracin_amd.scene import MODE_BEAUTY, MODE_NORMALS, make_view
+    heavy, light = (st.DeviceScene(st.gen_pbr(3, k), mesh_binned=True) for k in (30, 4))
+    implicit = st.DeviceScene(st.gen_implicit(3))
+    block = st.pinned_empty(48 << 20, np.uint32)
+    fake.act = None
+
+    def kernels(plain_mb, shaded):
+        """Primary kernels of a launch with plain images of so many MiB and Beauty requests (scene, million pixels)."""
+        w, h = 4096, round(plain_mb * 2**20 / 4 / 4096)
+        views, which, sizes = [make_view(width=w, height=h, mode=MODE_NORMALS)], [implicit], [w * h]
+        for ds, mpx in shaded:
+            h = round(mpx * 1e6 / 2048)
+            views.append(make_view(width=2047, height=h - 1, mode=MODE_BEAUTY, depth=2))
+            which.append(ds)
+            sizes.append(2047 * (h - 1))
+        at = np.concatenate([[0], np.cumsum(sizes)])
+        del fake.log[:]
+        st.render_batch_bgra8(which[::-1], np.concatenate(views[::-1]), outs=[block[at[i]:at[i + 1]] for i in range(len(sizes))][::-1])
+        return fake.log.count("launch k_primary4")
+
+    mb = 2**20 / 1e6
+    assert kernels(47.9, [(heavy, 2.0)]) == 1
+    assert kernels(48.1, [(heavy, 48.1 * mb / 32 + 0.01)]) == 2
+    assert kernels(60.0, [(heavy, 60.0 * mb / 32 - 0.01)]) == 1
+    assert kernels(60.0, [(light, 60.0 * mb / 20 - 0.01)]) == 1
+    assert kernels(60.0, [(light, 60.0 * mb / 20 + 0.01)]) == 2
+    assert kernels(60.0, [(light, 30.0 * mb / 20 + 0.01), (heavy, 30.0 * mb / 32 + 0.01)]) == 2
+    assert kernels(48.1, [(implicit, 16.0)]) == 1
+
+
 @pytest.fixture(scope="module")
 def fake_so(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
