@@ -319,6 +319,17 @@ def a_mesh_build_keeps_no_device_memory(fake, st):
         assert fake.so.fake_device_bytes() == with_server
         srv.close()
         assert fake.so.fake_device_bytes() == before
+    # a launch buffer that is large enough serves as scratch; one that is not stays as it is
+    from slimtracin_amd.scene import MODE_BEAUTY, make_view
+    for size, allocations in ((64, 2), (1600, 1)):
+        ds = st.DeviceScene(st.gen_implicit(3))
+        st.render(ds, make_view(width=size, height=size, mode=MODE_BEAUTY, depth=2))
+        ds.close()
+        before = fake.so.fake_device_bytes()
+        del fake.log[:]
+        st.DeviceScene(blob, mesh_lbvh=True).close()
+        assert fake.log.count("hipMalloc") == allocations, (size, fake.log)
+        assert fake.so.fake_device_bytes() == before
 
 
 @case
