@@ -123,25 +123,40 @@ static inline hipError_t copy_spans(hipStream_t stream, CopyRing *ring, CopySpan
     }
     copy_calls(true);
     if (e != hipSuccess || total < least || !copy_ring_ready(ring)) return plain();
-    std::vector<CopySpan> chunk;
+    /* Slot by slot, as many spans as fit: 60 images of 120 KB 1555 us (1610
+       with plain calls, 2030 with a slot and an event for each). */
+    struct Piece {
+        char *dev, *host;
+        uint32_t at, bytes, limit;   /* at: in the slot */
+    };
+    std::vector<Piece> piece;
+    std::vector<uint32_t> first;     /* chunk i: pieces first[i] to first[i + 1] */
     /* A chunk's state: `open` says that its slot may be moved by a thread (the
        download into it is done, or the upload before it has left it), `moved`
        that a thread has done so. Threads take chunks in order. */
     std::vector<std::atomic<uint32_t>> open, moved;
     std::vector<std::thread> team;
     try {
-        chunk.reserve(total / COPY_SLOT_BYTES + nspans);
+        uint32_t used = COPY_SLOT_BYTES;
         for (size_t k = 0; k < nspans; k++)
-            for (size_t at = 0; at < spans[k].bytes && !spans[k].direct; at += COPY_SLOT_BYTES)
-                chunk.push_back({spans[k].dev + at, spans[k].host + at,
-                                 std::min(spans[k].bytes - at, (size_t)COPY_SLOT_BYTES), spans[k].limit, false});
-        std::vector<std::atomic<uint32_t>>(chunk.size()).swap(open);
-        std::vector<std::atomic<uint32_t>>(chunk.size()).swap(moved);
+            for (size_t done = 0; done < spans[k].bytes && !spans[k].direct;) {
+                if (used >= COPY_SLOT_BYTES) {
+                    first.push_back((uint32_t)piece.size());
+                    used = 0;
+                }
+                const uint32_t n = (uint32_t)std::min(spans[k].bytes - done, (size_t)(COPY_SLOT_BYTES - used));
+                piece.push_back({spans[k].dev + done, spans[k].host + done, used, n, spans[k].limit});
+                used = (used + n + 255u) & ~255u;
+                done += n;
+            }
+        first.push_back((uint32_t)piece.size());
+        std::vector<std::atomic<uint32_t>>(first.size()).swap(open);
+        std::vector<std::atomic<uint32_t>>(first.size()).swap(moved);
         team.reserve(COPY_THREADS);
     } catch (const std::bad_alloc &) {
         return plain();
     }
-    const uint32_t chunks = (uint32_t)chunk.size();
+    const uint32_t chunks = (uint32_t)first.size() - 1u;
     for (uint32_t i = 0; i < chunks; i++) open[i] = moved[i] = 0;
     std::atomic<uint32_t> next(0), stop(0);
     auto work = [&]() {
@@ -153,9 +168,12 @@ static inline hipError_t copy_spans(hipStream_t stream, CopyRing *ring, CopySpan
                 std::this_thread::yield();
             }
             char *slot = ring->base + (size_t)(i % COPY_SLOTS) * COPY_SLOT_BYTES;
-            if (download) memcpy(chunk[i].host, slot, chunk[i].bytes);
-            else memcpy(slot, chunk[i].host, chunk[i].bytes);
-            if (chunk[i].limit && !words_below(chunk[i].host, chunk[i].bytes, chunk[i].limit)) over = 1;
+            for (uint32_t k = first[i]; k < first[i + 1]; k++) {
+                const Piece &p = piece[k];
+                if (download) memcpy(p.host, slot + p.at, p.bytes);
+                else memcpy(slot + p.at, p.host, p.bytes);
+                if (p.limit && !words_below(p.host, p.bytes, p.limit)) over = 1;
+            }
             moved[i].store(1, std::memory_order_release);
         }
     };
@@ -171,9 +189,12 @@ static inline hipError_t copy_spans(hipStream_t stream, CopyRing *ring, CopySpan
     };
     auto queue = [&](uint32_t i) {
         char *slot = ring->base + (size_t)(i % COPY_SLOTS) * COPY_SLOT_BYTES;
-        const hipError_t q =
-            download ? hipMemcpyAsync(slot, chunk[i].dev, chunk[i].bytes, hipMemcpyDeviceToHost, stream)
-                     : hipMemcpyAsync(chunk[i].dev, slot, chunk[i].bytes, hipMemcpyHostToDevice, stream);
+        hipError_t q = hipSuccess;
+        for (uint32_t k = first[i]; k < first[i + 1] && q == hipSuccess; k++) {
+            const Piece &p = piece[k];
+            q = download ? hipMemcpyAsync(slot + p.at, p.dev, p.bytes, hipMemcpyDeviceToHost, stream)
+                         : hipMemcpyAsync(p.dev, slot + p.at, p.bytes, hipMemcpyHostToDevice, stream);
+        }
         return q != hipSuccess ? q : hipEventRecord(ring->ev[i % COPY_SLOTS], stream);
     };
     if (download) {

@@ -76,3 +76,14 @@ def test_downloads_into_page_locked_memory_that_the_device_does_not_write(scene,
         _, hits, _ = st.render(scene, view, out=out)
         assert out.tobytes() == want.tobytes() and hits.tobytes() == want_hits.tobytes()
         assert (block[:at] == 0x5A).all() and (block[at + 24 * n:] == 0x5A).all()
+
+
+def test_many_small_downloads(scene):
+    """Pageable window images of odd sizes that share the ring's slots equal the page-locked ones."""
+    sizes = [(3 + 7 * i % 400, 150 + 11 * i % 300) for i in range(90)] + [(1, 1), (1201, 1000)]
+    views = np.concatenate([make_view(width=w, height=h, mode=MODE_DEPTH, position=(0.0, 7.0, -11.0), pitch=-0.2)
+                            for w, h in sizes])
+    want, _ = st.render_batch_bgra8([scene] * len(sizes), views, outs=st.pinned_split([w * h for w, h in sizes], np.uint32))
+    got, _ = st.render_batch_bgra8([scene] * len(sizes), views)
+    for i in range(len(sizes)):
+        assert np.array_equal(got[i], want[i]), sizes[i]

@@ -423,6 +423,39 @@ def launches_are_split_when_there_is_enough_to_render_meanwhile(fake, st):
     assert kernels(48.1, [(implicit, 16.0)]) == 1
 
 
+@case
+def small_spans_share_the_slots_of_the_copy_ring(fake, st):
+    """Many small pageable outputs of one launch go slot by slot (2 MiB, an event each), and each arrives whole."""
+    import numpy as np
+    from slimtracin_amd.scene import MODE_DEPTH, make_view
+    ds = st.DeviceScene(st.gen_implicit(3))
+    sizes = [(3 + 7 * i % 400, 150 + 11 * i % 300) for i in range(90)] + [(1, 1), (1201, 1000)]
+    views = np.concatenate([make_view(width=w, height=h, mode=MODE_DEPTH) for w, h in sizes])
+    sent = []
+
+    def act(name, args):   # the device's bytes of each copy: its number
+        if name == "hipMemcpyAsync":
+            C.memset(args[1], len(sent) % 251 + 1, args[2])
+            sent.append(args[2])
+
+    outs = [np.zeros(w * h, np.uint32) for w, h in sizes]
+    st.render_batch_bgra8([ds] * len(sizes), views, outs=outs)
+    fake.act = act
+    del fake.log[:]
+    st.render_batch_bgra8([ds] * len(sizes), views, outs=outs)
+    total = sum(4 * w * h for w, h in sizes)
+    assert sum(sent) == total > 8 << 20
+    assert fake.log.count("hipEventRecord") <= total // (2 << 20) + 2, fake.log.count("hipEventRecord")
+    at = 0
+    for o in outs:
+        b, done = o.view(np.uint8), 0
+        while done < len(b):
+            assert (b[done:done + sent[at]] == at % 251 + 1).all(), at
+            done += sent[at]
+            at += 1
+    assert at == len(sent)
+
+
 @pytest.fixture(scope="module")
 def fake_so(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
