@@ -46,7 +46,8 @@ def _blob():
 VIEWS = [
     dict(position=(0.0, 3.0, -10.0), width=33, height=21),
     dict(position=(0.0, 3.0, -10.0), width=65, height=49),
-    dict(position=(-10.0, 3.0, 0.0), yaw=1.0, width=45, height=27),
+    dict(position=(-10.0, 3.0, 0.0), yaw=1.0, width=45, height=27),   # looks away from the mesh
+    dict(position=(10.0, 3.0, 0.0), yaw=1.0, width=45, height=27),    # at it
 ]
 
 
@@ -82,6 +83,8 @@ def test_views_hold_zero_direction_components(k):
     axes = {c for _, _, c in zeros}
     assert zeros, "no degenerate ray in the view"
     assert axes == ({0, 1} if k < 2 else {1, 2}), axes
+    steps = ck.oracle_render_steps(blob, view)[2]
+    assert (steps.max() > 1000) == (k != 2), steps.max()   # such rays through the mesh, and their long traversals
 
 
 @pytest.mark.skipif(not ck.ref_available(), reason="reference build missing")
