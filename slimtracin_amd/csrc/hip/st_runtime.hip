@@ -1093,8 +1093,8 @@ __global__ void __launch_bounds__(256) k_ssb(const StDScene *__restrict__ scenes
 /* Everything the primary stage needs of a launch besides its upload, in one
    launch: the primary directions (the longest: a row's additions are one
    chain, 19 us for 1920), the tile order and the SSB rects, each by its own
-   run of blocks. As three launches one after another they and the gaps
-   between them took PREPB. */
+   run of blocks, so that the short ones run beside the chains: 22 us for a
+   1920x1080 frame, 29 as three launches (20, 4 and 5). */
 __global__ void __launch_bounds__(PREP_THREADS) k_prep(const StDScene *__restrict__ scenes,
                                                        const KReq *__restrict__ reqs, uint32_t nreq,
                                                        uint32_t total_rows, uint32_t dir_blocks,
@@ -1573,7 +1573,7 @@ static int build_device_meshes(StSceneHandle *h) {
     }
     if (!any) return ST_OK;
     /* a build's scratch: the main context's launch buffer where that is large
-       enough as it is (about 400 MB after a 1920x1080 Beauty frame), else
+       enough as it is (about 0.5 GB after a 1920x1080 Beauty frame), else
        memory that is gone when the scene is there: its allocation and release
        take 0.05 to 0.35 ms (3.7 ms is what admitting 1,000,000 triangles
        takes). The launch buffer does not grow for a build: a server's launches
@@ -2004,10 +2004,11 @@ static Switches switches_now(void) {
 
 /* Upload and run one launch on context c over `n` requests whose host views
    are already prepared (camera basis, row starts, SSB rects). Each
-   request's frame (and hit records) is copied to pixels_host[i] /
-   hits_host[i] when given. Returns when the launch is done. Runs without
-   the library lock on a server context: only c's own buffers are written,
-   the scenes are read. The first `plain` requests have no bounce stage and are
+   request's frame, hit records and window image go to pixels_host[i],
+   hits_host[i] and bgra_host[i] when given: written there by the device
+   (deliverable), or copied after the last kernel. Returns when the launch is
+   done. Runs without the library lock on a server context: only c's own
+   buffers and the outputs are written, the scenes are read. The first `plain` requests have no bounce stage and are
    delivered early (KEarly). apart: no two outputs overlap. */
 static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const *scenes, StHostView *hv, uint32_t n,
                           uint32_t plain, bool apart, int want_hits, int persistent, StRayCounts *counts,
@@ -2020,7 +2021,7 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
     std::vector<StSceneHandle *> uniq(n);
     uint32_t nuniq = 0;
     /* one upload block (requests, scene table, row starts, rects), staged in
-       pinned memory and copied with a single transfer */
+       page-locked memory, from where k_setup takes it */
     std::vector<size_t> rs_off(n), rect_off(n);
     size_t up = round256(n * sizeof(KReq));
     size_t per_req_out = 0;
@@ -2588,8 +2589,8 @@ extern "C" int st_render(StSceneHandle *scene, const StView *view, StFloatPixel 
 }
 
 /* st_render without allocating: every per-launch device buffer is carved
-   from this device's scratch array, the host side uses static buffers, and
-   the launch runs on the main stream. The same kernels, in the same order,
+   from this device's scratch array, the host side uses page-locked memory
+   that st_init took, and the launch runs on the main stream. The same kernels, in the same order,
    as a single-request st_render (tiles in tile order: the array keeps no
    tile history). */
 extern "C" int st_render_noalloc(StSceneHandle *scene, const StView *view, StFloatPixel *pixels, StHitRec *hits,

@@ -6,8 +6,8 @@
  * buffers, pinned staging): a free worker takes everything queued (up to
  * the batch limits), prepares each request's camera set-up on the host and
  * runs the batch as one persistent launch on its context (one tile list over
- * all requests, one upload transfer, device display resolve, downloads into
- * pinned per-ticket buffers). Requests that arrive while launches run are
+ * all requests, one upload, device display resolve straight into the
+ * page-locked per-ticket buffers). Requests that arrive while launches run are
  * taken by the next free worker and launched at once on its own stream, so
  * their work overlaps on the device with the launches already there; a
  * launch that runs long holds only its own requests. Scenes are admitted
