@@ -1374,7 +1374,10 @@ static int ctx_init(LaunchCtx *c) {
     HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIP_TRY(hipMalloc(&c->tile_counter, CLAIM_WORDS * sizeof(uint32_t)));
     HIP_TRY(hipMalloc(&c->cost_sum, 256));
-    HIP_TRY(hipMemset(c->cost_sum, 0, 256));
+    /* cleared on the context's own stream: hipMemset returns before its fill
+       (on the null stream) is done, and nothing orders that before launches here */
+    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, c->stream, (uint32_t *)c->cost_sum, 64u);
+    HIP_TRY(hipGetLastError());
     for (int i = 0; i < 4; i++) HIP_TRY(hipEventCreate(&c->ev[i]));
     return ST_OK;
 }
@@ -2143,7 +2146,11 @@ static int launch_ordered(LaunchCtx *c, const Switches &sw, StSceneHandle *const
         c->tile_cap = 0;
         c->tile_sig = 0;
         HIP_TRY(hipMalloc(&c->tile_cost, (size_t)tiles * 8));
-        HIP_TRY(hipMemset(c->tile_cost, 0, (size_t)tiles * 8));
+        /* (on this stream, as in ctx_init: a late fill would clear the claim
+           order of a launch that has begun, and tiles would stay unrendered) */
+        hipLaunchKernelGGL(k_zero_u32, dim3((2u * tiles + 255u) / 256u), dim3(256), 0, c->stream, c->tile_cost,
+                           2u * tiles);
+        HIP_TRY(hipGetLastError());
         c->tile_order = c->tile_cost + tiles;
         c->tile_cap = tiles;
     }

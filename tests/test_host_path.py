@@ -338,6 +338,7 @@ def a_timed_launch_is_timed_from_its_upload_on(fake, st):
     from slimtracin_amd.scene import MODE_BEAUTY, make_view
     ds = st.DeviceScene(st.gen_pbr(3, 10))
     view = make_view(width=90, height=70, mode=MODE_BEAUTY, depth=3)
+    st.render(ds, view)   # the context's arrays are there
     for stages in (False, True):
         for graph in (False, True):
             for _ in range(2):
@@ -454,6 +455,32 @@ def small_spans_share_the_slots_of_the_copy_ring(fake, st):
             done += sent[at]
             at += 1
     assert at == len(sent)
+
+
+@case
+def nothing_is_filled_behind_a_launchs_back(fake, st):
+    """hipMemset returns before its fill is done, on a stream that nothing orders against a context's own: a context's
+    words and tile arrays are cleared by kernels on its stream, before the launch that uses them."""
+    from slimtracin_amd.scene import MODE_BEAUTY, make_view
+    from slimtracin_amd.server import Server
+    blob = st.gen_implicit(3)
+    ds = st.DeviceScene(blob)
+    srv = Server(max_in_flight=2)
+    sid = srv.add_scene(blob)
+    assert fake.log.count("launch k_zero_u32") == 3, fake.log   # the main context and the server's two
+    for size in (64, 900, 300, 1200):
+        view = make_view(width=size, height=size, mode=MODE_BEAUTY, depth=2)
+        del fake.log[:]
+        st.render(ds, view)
+        grown = fake.log.count("launch k_zero_u32")
+        assert grown == (size != 300), fake.log
+        if grown:
+            assert fake.log.index("launch k_zero_u32") < fake.log.index("launch k_setup")
+        t = srv.submit(sid, view)
+        srv.wait(t, copy=False)
+        srv.release(t)
+        assert "hipMemset" not in fake.log, fake.log
+    srv.close()
 
 
 @pytest.fixture(scope="module")
