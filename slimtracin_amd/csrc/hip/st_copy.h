@@ -24,13 +24,16 @@
 
 #define COPY_SLOTS 8u
 #define COPY_SLOT_BYTES (2u << 20)
-/* Bytes from which the ring is the quicker. A depth frame into pageable
-   memory, ring and call: 2 MiB 216 and 178 us, 3 MiB 269 and 257, 4 MiB 314
-   and 328, 8 MiB 460 and 605. Creating a scene with a device-built mesh (its
-   geometry checked by the threads, or on one): 11.9 MB 1010 and 922 us, 15.9
-   MB 1155 and 1070, 31.8 MB 2075 and 2300, 49.6 MB 2765 and 3515. */
-#define COPY_MIN_DOWNLOAD (4u << 20)
-#define COPY_MIN_UPLOAD (24u << 20)
+/* Bytes from which the ring is used. A depth frame into pageable memory, ring
+   and call: 2 MiB 216 and 178 us, 3 MiB 269 and 257, 4 MiB 314 and 328, 8 MiB
+   460 and 605. Uploads by themselves gain from some 20 MB on (creating a scene
+   with a device-built mesh: 11.9 MB 1010 and 922 us, 15.9 MB 1155 and 1070,
+   31.8 MB 2075 and 2300, 49.6 MB 2765 and 3515), but a large call leaves the
+   caller's memory known to the runtime, and the launches that follow pay when
+   that memory is freed: the first burst of 48 requests at a new server with
+   four scenes of 22 MB took 13.2 ms (15.1 in one of 8 processes) with their
+   uploads through the ring, and 16.5 in 5 of 8 with calls. */
+#define COPY_MIN_BYTES (4u << 20)
 #define COPY_THREADS 8u
 
 /* A launch context's ring: 16 MiB of page-locked memory and an event per
@@ -94,7 +97,6 @@ static inline bool copy_known(const char *p) {
    themselves, on one thread: 2 ms). */
 static inline hipError_t copy_spans(hipStream_t stream, CopyRing *ring, CopySpan *spans, size_t nspans,
                                        bool download, bool in_order, bool *in_range = nullptr) {
-    const size_t least = download ? COPY_MIN_DOWNLOAD : COPY_MIN_UPLOAD;
     size_t total = 0;
     for (size_t k = 0; k < nspans; k++) total += spans[k].bytes;
     std::atomic<uint32_t> over(0);
@@ -115,14 +117,14 @@ static inline hipError_t copy_spans(hipStream_t stream, CopyRing *ring, CopySpan
     };
     if (in_range) *in_range = true;
     for (size_t k = 0; k < nspans; k++) spans[k].direct = false;
-    if (in_order || total < least) return plain();
+    if (in_order || total < COPY_MIN_BYTES) return plain();
     for (size_t k = 0; k < nspans; k++) {
         CopySpan &s = spans[k];
         s.direct = s.bytes && !s.limit && copy_known(s.host) && copy_known(s.host + s.bytes - 1);
         if (s.direct) total -= s.bytes;
     }
     copy_calls(true);
-    if (e != hipSuccess || total < least || !copy_ring_ready(ring)) return plain();
+    if (e != hipSuccess || total < COPY_MIN_BYTES || !copy_ring_ready(ring)) return plain();
     /* Slot by slot, as many spans as fit: 60 images of 120 KB 1555 us (1610
        with plain calls, 2030 with a slot and an event for each). */
     struct Piece {

@@ -38,7 +38,7 @@ def test_downloads(scene, w, h):
         assert np.array_equal(hits["prim_id"] >= 0, np.isfinite(want["depth"]))
 
 
-@pytest.mark.parametrize("tris", [500, 200_000, 600_000])   # 600,000: through the ring
+@pytest.mark.parametrize("tris", [500, 200_000, 600_000])
 @pytest.mark.parametrize("which", ["position", "normal"])
 @pytest.mark.parametrize("place", ["first", "middle", "last"])
 def test_indices_out_of_range_are_refused(tris, which, place):

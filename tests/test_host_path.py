@@ -285,12 +285,12 @@ def page_locked_memory_of_others_is_copied_directly(fake, st):
 
 @case
 def only_large_copies_take_threads(fake, st):
-    """Uploads below 24 MiB and downloads below 4 MiB are plain calls, on the calling thread."""
+    """Copies below 4 MiB are plain calls, on the calling thread."""
     from slimtracin_amd.scene import MODE_DEPTH, make_view
     threads = []
     fake.act = lambda name, args: threads.append(_threads())
     before = _threads()
-    for triangles, ring in ((400000, False), (600000, True)):
+    for triangles, ring in ((60000, False), (100000, True)):
         blob = st.gen_mesh_scene(3, triangles)
         del threads[:]
         st.DeviceScene(blob, mesh_lbvh=True).close()
