@@ -28,11 +28,11 @@
    and call: 2 MiB 216 and 178 us, 3 MiB 269 and 257, 4 MiB 314 and 328, 8 MiB
    460 and 605. Uploads by themselves gain from some 20 MB on (creating a scene
    with a device-built mesh: 11.9 MB 1010 and 922 us, 15.9 MB 1155 and 1070,
-   31.8 MB 2075 and 2300, 49.6 MB 2765 and 3515), but a large call leaves the
-   caller's memory known to the runtime, and the launches that follow pay when
-   that memory is freed: the first burst of 48 requests at a new server with
-   four scenes of 22 MB took 13.2 ms (15.1 in one of 8 processes) with their
-   uploads through the ring, and 16.5 in 5 of 8 with calls. */
+   31.8 MB 2075 and 2300, 49.6 MB 2765 and 3515), but the launches after large
+   calls pay for them, it seems where the caller's memory, pinned for the call,
+   is freed: the first burst of 48 requests at a new server with four scenes of
+   22 MB took 13.2 ms (15.1 in one of 8 processes) with their uploads through
+   the ring, and 16.5 in 5 of 8 with calls. */
 #define COPY_MIN_BYTES (4u << 20)
 #define COPY_THREADS 8u
 
